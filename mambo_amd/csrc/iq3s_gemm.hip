@@ -29,7 +29,9 @@
 // M up to 4 per MFMA, up to 16 per pass (U = 1..4 MFMAs per K step).
 #include <mutex>
 
+#include "iq3s_dense.h"
 #include "iq3s_stream.h"
+#include "iq3s_wide.h"
 
 namespace {
 
@@ -288,51 +290,6 @@ __device__ __forceinline__ void load_a_dense_rsrc(ADense &at, __amdgpu_buffer_rs
         at.a[h] = v8i{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
         at.s[h] = __builtin_amdgcn_raw_buffer_load_b8(sr, soff + h, 8u * b, 0);
     }
-}
-
-// hi and lo words of code C of a group: level bytes select from the split table entry
-// (tab.x/.y: hi of levels 0-3/4-7, tab.z/.w: lo); the four signs, moved onto bits
-// 7,15,23,31 by one shift of the transposed sign word, are OR-ed into hi and XOR-ed into
-// lo (one v_bitop3 each: a | (b & c) = 0xF8, a ^ (b & c) = 0x78).
-template <int C>
-__device__ __forceinline__ void split_word(uint32_t lv, uint32_t p, uint4 tab, int &hi, int &lo)
-{
-    const uint32_t r = funnel_shr(p, p, (25 + C) & 31);
-    hi = (int)__builtin_amdgcn_bitop3_b32(__builtin_amdgcn_perm(tab.y, tab.x, lv), r, 0x80808080u, 0xF8);
-    lo = (int)__builtin_amdgcn_bitop3_b32(__builtin_amdgcn_perm(tab.w, tab.z, lv), r, 0x80808080u, 0x78);
-}
-
-// Split-table entry of operand half X (0: bytes 0-15, 1: bytes 16-31) of MFMA H, from the
-// lane's dense scale word (dense_scales: nibble 2X + H).
-template <int H, int X>
-__device__ __forceinline__ uint4 split_entry(const uint4 *split, uint32_t sc)
-{
-    return split[(sc >> (4 * (2 * X + H))) & 15u];
-}
-
-// MFMA H's hi and lo operands: codes 0-3 with the entry of half 0 (ta), 4-7 of half 1 (tb).
-template <int H, int... C>
-__device__ __forceinline__ void decode_split(const uint32_t (&s)[5], uint32_t p, const uint8_t *lvl, uint4 ta,
-                                             uint4 tb, v8i &bhi, v8i &blo, std::integer_sequence<int, C...>)
-{
-    int h[8], l[8];
-    (split_word<C>(*reinterpret_cast<const uint32_t *>(lvl + code_addr<8 * H + C>(s)), p, C < 4 ? ta : tb, h[C],
-                   l[C]),
-     ...);
-    bhi = v8i{h[0], h[1], h[2], h[3], h[4], h[5], h[6], h[7]};
-    blo = v8i{l[0], l[1], l[2], l[3], l[4], l[5], l[6], l[7]};
-}
-
-// Both halves of one tile-block (MFMA H = 0, 1).
-__device__ __forceinline__ void decode_block(const WTile &w, const uint8_t *lvl, const uint4 *split, v8i (&bh)[2],
-                                             v8i (&bl)[2])
-{
-    const uint32_t s[5] = {w.ia.x, w.ia.y, w.ia.z, w.ia.w, (uint32_t)w.ib};
-    const uint32_t sc = dense_scales(w.sc);
-    decode_split<0>(s, w.sg.x, lvl, split_entry<0, 0>(split, sc), split_entry<0, 1>(split, sc), bh[0], bl[0],
-                    std::make_integer_sequence<int, 8>{});
-    decode_split<1>(s, w.sg.y, lvl, split_entry<1, 0>(split, sc), split_entry<1, 1>(split, sc), bh[1], bl[1],
-                    std::make_integer_sequence<int, 8>{});
 }
 
 template <int MC>
@@ -1980,6 +1937,25 @@ int plan_streaming(const mambo_gemm_config &c, const uint8_t *xv, int64_t ldxv, 
 }
 
 
+// Whether a configuration names nothing (the library chooses).
+bool all_default(const mambo_gemm_config &c)
+{
+    return c.kernel == MAMBO_GEMM_AUTO && c.waves == 0 && c.split_k == 0 && c.tile_m == 0 && c.tile_n == 0;
+}
+
+// Zero fill of a K split's accumulators, every projection's output in one dispatch.
+int zero_outputs(const GroupArgs &ga, int64_t m, hipStream_t s)
+{
+    int64_t n_max = 0;
+    for (int g = 0; g < ga.count; ++g)
+        n_max = std::max(n_max, ga.n[g]);
+    const int64_t chunks = m * cdiv(n_max, 4); // 4-float chunks of the widest projection
+    MAMBO_REQUIRE(chunks <= 0x7FFFFFFF, MAMBO_ERR_VALUE, "output too large for one split-K launch");
+    const dim3 grid((unsigned)std::min<int64_t>(cdiv(chunks, 256), 1024), (unsigned)ga.count);
+    MAMBO_LAUNCH(zero_rows_kernel, grid, dim3(256), 0, s, ga, (int)m);
+    return mambo_check_launch("zero_rows");
+}
+
 // quant: -1 when xv/xs are MXFP8 activations; else xv holds unquantized rows of dtype
 // quant (ldxv in elements, xs unused) for the stream kernel to quantize itself, and the
 // call returns kNotFused, launching nothing, when the configuration cannot do that.
@@ -2037,6 +2013,18 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
         if (rc)
             return rc;
     }
+    // A call that leaves the configuration to the library takes the 32 x 32 MFMA kernel where
+    // that is the faster one.
+    WidePlan wide;
+    if (quant < 0 && (cfg == nullptr || all_default(*cfg)) &&
+        mambo_wide_plan(m, proj, count, blocks, ldxv, xs, ldxs, c, &wide)) {
+        if (wide.splits > 1) {
+            rc = zero_outputs(ga, m, s);
+            if (rc)
+                return rc;
+        }
+        return mambo_wide_launch(wide, xv, ldxv, xs, ldxs, m, proj, count, blocks, s);
+    }
     if (quant >= 0) { // in-kernel quantization: stream kernel, one sub-tile, rows staged in LDS
         const int64_t esz = quant == MAMBO_DTYPE_BF16 ? 2 : 4;
         const int qrows = (int)std::min<int64_t>(4, m);
@@ -2088,14 +2076,7 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
     if (rc)
         return rc;
     if (atomic) {
-        int64_t n_max = 0;
-        for (int g = 0; g < count; ++g)
-            n_max = std::max(n_max, ga.n[g]);
-        const int64_t chunks = m * cdiv(n_max, 4); // 4-float chunks of the widest projection
-        MAMBO_REQUIRE(chunks <= 0x7FFFFFFF, MAMBO_ERR_VALUE, "output too large for one split-K launch");
-        dim3 zg((unsigned)std::min<int64_t>(cdiv(chunks, 256), 1024), (unsigned)count);
-        MAMBO_LAUNCH(zero_rows_kernel, zg, dim3(256), 0, s, ga, (int)m);
-        rc = mambo_check_launch("zero_rows");
+        rc = zero_outputs(ga, m, s);
         if (rc)
             return rc;
     }

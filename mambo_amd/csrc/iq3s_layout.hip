@@ -271,6 +271,14 @@ __global__ __launch_bounds__(256) void pack_fields_kernel(SoaSrc src, int64_t n,
         pack_lane(FieldBlock{src, b * n + row, row < n}, lane, packed + (t * blocks + b) * (int64_t)kTileBytes);
 }
 
+// 32 rows x kBlocks blocks per workgroup, one weight group (32 values) per thread and block: of a
+// block the workgroup reads contiguous runs of the fields (2 KiB of qs) and writes 32 whole
+// 256-byte pieces, where a thread per group along a row read 64 bytes of qs here and there.
+// Memory-bound (110 bytes in, 288 out per block), so all loads of the blocks come first.
+// 4096 x 14336: 25 -> 17.6 us, 28672 x 4096: 38.5 -> 31.5 us (5.8 TB/s; a copy moves 4.8), level
+// below 1024 x 8192. Nontemporal stores are slower (63 us at 28672 x 4096).
+constexpr int kDequantRows = 32;
+template <int kBlocks>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict__ d, const uint32_t *__restrict__ qs,
                                                       const uint16_t *__restrict__ qh,
                                                       const int32_t *__restrict__ signs,
@@ -282,31 +290,42 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict
     for (int i = threadIdx.x; i < 512; i += blockDim.x)
         lut[i] = c_grid.fp8[i];
     __syncthreads();
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t total = n * blocks * 8;
-    if (gid >= total)
+    const int g = (int)threadIdx.x & 7;
+    const int64_t row = (int64_t)blockIdx.x * kDequantRows + (threadIdx.x >> 3);
+    if (row >= n)
         return;
-    const int g = (int)(gid & 7);
-    const int64_t b = (gid >> 3) % blocks;
-    const int64_t row = (gid >> 3) / blocks;
-    const int64_t e = b * n + row;
-    const uint32_t q0 = qs[e * 16 + 2 * g], q1 = qs[e * 16 + 2 * g + 1];
-    const uint32_t hb = reinterpret_cast<const uint8_t *>(qh)[e * 8 + g];
-    const uint32_t sw = (uint32_t)signs[e * 8 + g];
-    const uint32_t s = (scales[e] >> (4 * g)) & 15u;
-    uint32_t out[8];
+    for (int64_t b0 = (int64_t)blockIdx.y * kBlocks; b0 < blocks; b0 += (int64_t)gridDim.y * kBlocks) {
+        uint2 q[kBlocks];
+        uint32_t hb[kBlocks], sw[kBlocks], sc[kBlocks];
+        uint16_t db[kBlocks];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const uint32_t lo = ((c < 4 ? q0 : q1) >> (8 * (c & 3))) & 0xFFu;
-        const uint32_t idx = lo | (((hb >> c) & 1u) << 8);
-        const uint32_t nib = (sw >> (4 * c)) & 15u;
-        const uint32_t mask = ((nib & 1u) << 7) | ((nib & 2u) << 14) | ((nib & 4u) << 21) | ((nib & 8u) << 28);
-        out[c] = lut[idx] | mask;
+        for (int j = 0; j < kBlocks; ++j) { // all loads first; past the weight the last block again
+            const int64_t e = min(b0 + j, blocks - 1) * n + row;
+            q[j] = make_uint2(qs[e * 16 + 2 * g], qs[e * 16 + 2 * g + 1]);
+            hb[j] = reinterpret_cast<const uint8_t *>(qh)[e * 8 + g];
+            sw[j] = (uint32_t)signs[e * 8 + g];
+            sc[j] = scales[e];
+            db[j] = d[e];
+        }
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) {
+            const int64_t b = b0 + j;
+            if (b >= blocks)
+                break;
+            uint32_t out[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const uint32_t idx = (((c < 4 ? q[j].x : q[j].y) >> (8 * (c & 3))) & 0xFFu) | (((hb[j] >> c) & 1u) << 8);
+                const uint32_t nib = (sw[j] >> (4 * c)) & 15u;
+                out[c] = lut[idx] | ((nib * 0x00204081u & 0x01010101u) << 7);
+            }
+            uint4 *vp = reinterpret_cast<uint4 *>(values + (row * blocks + b) * 256 + 32 * g);
+            vp[0] = make_uint4(out[0], out[1], out[2], out[3]);
+            vp[1] = make_uint4(out[4], out[5], out[6], out[7]);
+            out_scales[(row * blocks + b) * 8 + g] =
+                half_bits_to_float(db[j]) * (float)(1u + 2u * ((sc[j] >> (4 * g)) & 15u));
+        }
     }
-    uint4 *vp = reinterpret_cast<uint4 *>(values + row * blocks * 256 + b * 256 + 32 * g);
-    vp[0] = make_uint4(out[0], out[1], out[2], out[3]);
-    vp[1] = make_uint4(out[4], out[5], out[6], out[7]);
-    out_scales[row * blocks * 8 + b * 8 + g] = half_bits_to_float(d[e]) * (float)(1u + 2u * s);
 }
 
 } // namespace
@@ -372,7 +391,13 @@ extern "C" int mambo_iq3s_dequant(const uint16_t *d, const uint32_t *qs, const u
     MAMBO_REQUIRE((uintptr_t)values % 16 == 0, MAMBO_ERR_VALUE, "values must be 16-byte aligned");
     const int64_t total = n * blocks * 8;
     MAMBO_REQUIRE((total + 255) / 256 <= 0x7FFFFFFF, MAMBO_ERR_VALUE, "weight too large");
-    MAMBO_LAUNCH(dequant_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, d,
-                       qs, qh, signs, scales, n, blocks, values, out_scales);
+    // a single block per workgroup where four would leave CUs idle (1024 x 4096: 4.4 us with four,
+    // 3.7 with one; 4096 x 4096, 512 workgroups: 7.3 and 7.9; level from 6144 x 8192 on)
+    const int64_t rows = (n + kDequantRows - 1) / kDequantRows;
+    const bool four = rows * ((blocks + 3) / 4) >= 512;
+    const int64_t groups = four ? (blocks + 3) / 4 : blocks;
+    const dim3 grid((unsigned)rows, (unsigned)(groups < 65535 ? groups : 65535));
+    MAMBO_LAUNCH(four ? dequant_kernel<4> : dequant_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, d, qs, qh, signs, scales, n, blocks, values,
+                 out_scales);
     return mambo_check_launch("iq3s_dequant");
 }

@@ -1,5 +1,5 @@
 """Weight preparation and decoding at the edges of their workgroups (64 rows x 4 blocks or a tile;
-one weight group a thread), from every form of source: whole fields against numpy, bit for bit,
+32 rows x 1 or 4 blocks), from every form of source: whole fields against numpy, bit for bit,
 and the tile layout against the one that the byte path builds."""
 
 from __future__ import annotations

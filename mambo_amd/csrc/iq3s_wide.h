@@ -5,7 +5,8 @@
 // Launch shape of gemm_wide_kernel for one call.
 struct WidePlan {
     int mt;     // 32-token sub-tiles per workgroup
-    int waves;  // per workgroup, 32 weight rows each
+    int waves;  // per K group, 32 weight rows each
+    int kg;     // K groups of waves per workgroup
     int splits; // K slices (more than one: f32 atomics into outputs zeroed beforehand)
     int bps;    // K blocks per slice
 };

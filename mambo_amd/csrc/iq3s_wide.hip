@@ -1,7 +1,8 @@
 // Projection for 33 tokens and more on V_MFMA_SCALE_F32_32X32X64_F8F6F4.
 //
-// A workgroup of W waves computes 32*MT tokens x 32*W weight rows; a wave owns two 16-row
-// weight tiles (32 rows) and MT sub-tiles of 32 tokens. As in the tiled kernel
+// A workgroup computes 32*MT tokens x 32*W weight rows with KG groups of W waves, each group
+// taking a KG-th of the workgroup's K blocks; a wave owns two 16-row weight tiles (32 rows) and
+// MT sub-tiles of 32 tokens. As in the tiled kernel
 // (iq3s_gemm.hip) the block's activations are copied straight into double-buffered LDS, the
 // weights are the exact two-term E4M3 operands of iq3s_dense.h, a block's sums are one MFMA
 // chain (four K steps of 64 x hi/lo) and the block's fp16 d is applied in f32.
@@ -23,6 +24,14 @@
 // decoded (a second block in flight measured no faster). 230 VGPRs at MT = 4, so two waves
 // per SIMD; what bounds it there is the power limit (1.7 GHz at 55% MFMA busy at 8192 tokens)
 // and, up to a few hundred tokens, the latency of a step's dependent chain.
+//
+// Two K groups (their sums meet in LDS at the end) put two waves on each SIMD where a launch
+// has a workgroup per CU or less: one wave leaves its SIMD idle while a step's chain of LDS
+// reads, decode and MFMAs completes (1.26 us a block of 64 tokens against 1.82 for two waves'),
+// and a K split over half as many workgroups costs half the atomics. One group against two,
+// each at its fastest split (us): 28672 x 4096 at 48 tokens 29 -> 25.6, 10240 x 8192 at 256
+// 59 -> 51, 6144 x 4096 at 256 25 -> 22, 8192 x 28672 at 128 80 -> 72, 4096 x 14336 at 256
+// 54 -> 43. Launches that fill the chip gain nothing from it (57344 x 8192 at 48: 82 and 85).
 //
 // Measured against the kernels it takes over from, same box, one launch in a replayed graph
 // over rotated weights (us): 57344 x 8192 at 40 / 128 / 512 tokens 133 -> 77, 133 -> 109, 456 ->
@@ -114,8 +123,8 @@ __device__ __forceinline__ void finish_words(const WState &st, const uint32_t (&
 
 // kPolicy: cache policy of the weight loads, non-temporal where one token tile reads each
 // weight once (57344 x 8192 at 128 tokens 0-2%), the default where several do.
-template <int MT, int W, int kPolicy>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_wide_kernel(
+template <int MT, int W, int KG, int kPolicy>
+__global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_wide_kernel(
     const uint8_t *__restrict__ xv, int64_t ldxv, const uint8_t *__restrict__ xs, int64_t ldxs, int64_t M, GroupArgs ga,
     int B, int bps, int atomic)
 {
@@ -128,12 +137,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
     // more vector instructions per block, 3-5% of the kernel)
     __shared__ __align__(1024) uint32_t s_lvl[512];
     __shared__ __align__(256) uint4 s_split[16];
-    __shared__ __align__(128) uint8_t s_scale0[kRows * 8];
-    __shared__ __align__(128) uint8_t s_scale1[kRows * 8];
-    __shared__ __align__(16) uint8_t s_vals0[kRows * 256];
-    __shared__ __align__(16) uint8_t s_vals1[kRows * 256];
+    __shared__ __align__(128) uint8_t s_scale0[KG * kRows * 8];
+    __shared__ __align__(128) uint8_t s_scale1[KG * kRows * 8];
+    __shared__ __align__(16) uint8_t s_vals0[KG * kRows * 256];
+    __shared__ __align__(16) uint8_t s_vals1[KG * kRows * 256];
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wgwave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wgwave % W, kg = wgwave / W; // wave within its K group
     const int col = lane & 15, r32 = lane & 31, g = lane >> 5;
 
     const uint8_t *packed = ga.packed[0];
@@ -171,8 +181,8 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
                           16u * (uint32_t)((lane & 15) ^ ((4 * wave + (lane >> 4)) & 15));
     const uint32_t soff_stage = (uint32_t)(32 * srow + (lane >> 1)) * (uint32_t)ldxs + 4u * (lane & 1);
 
-    const uint32_t a0 = 256u * r32 + 16u * (uint32_t)(g ^ col);
-    const uint32_t soff = 8u * r32 + 2u * g;
+    const uint32_t a0 = (uint32_t)(kg * kRows * 256) + 256u * r32 + 16u * (uint32_t)(g ^ col);
+    const uint32_t soff = (uint32_t)(kg * kRows * 8) + 8u * r32 + 2u * g;
     const uint8_t *lvl = reinterpret_cast<const uint8_t *>(s_lvl);
 
     float acc[MT][16];
@@ -182,15 +192,17 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
         for (int i = 0; i < 16; ++i)
             acc[mt][i] = c[mt][i] = 0.0f;
-    const int b0 = blockIdx.z * bps, b1 = min(B, b0 + bps);
+    // K group kg takes blocks [b0, end); those from b1 on count with a zero d
+    const int z0 = blockIdx.z * bps, b1 = min(B, z0 + bps), per = (b1 - z0 + KG - 1) / KG;
+    const int b0 = z0 + kg * per, end = b0 + per;
     auto wblock = [&](int b) { return (uint32_t)min(b, b1 - 1) * kTileBytes; };
 
     auto stage = [&](uint8_t *vals, uint8_t *scl, int b) {
 #pragma unroll
         for (int j = 0; j < kVCopies; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrows, (lds_ptr)(vals + 1024 * (wave + W * j)), 16, voff,
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrows, (lds_ptr)(vals + kg * kRows * 256 + 1024 * (wave + W * j)), 16, voff,
                                                      256u * b + (uint32_t)(4 * W * j) * (uint32_t)ldxv, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(srows, (lds_ptr)(scl + 256 * srow), 4, soff_stage, 8u * b, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(srows, (lds_ptr)(scl + kg * kRows * 8 + 256 * srow), 4, soff_stage, 8u * b, 0, 0);
     };
 
     WRec rec[2];
@@ -204,14 +216,14 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
     // for the copies only (vector memory completes in issue order).
     {
         const __amdgpu_buffer_rsrc_t gr = byte_rsrc(c_grid.level), tr = byte_rsrc(&c_split.w[0][0]);
-        for (int i = wave; i < 9; i += W) {
+        for (int i = wgwave; i < 9; i += W * KG) {
             if (i < 8)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(gr, (lds_ptr)(s_lvl + 64 * i), 4, 4u * lane, 256u * i, 0, 0);
             else
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(tr, (lds_ptr)s_split, 4, 4u * lane, 0, 0, 0);
         }
     }
-    stage(s_vals0, s_scale0, b0);
+    stage(s_vals0, s_scale0, min(b0, b1 - 1));
     __builtin_amdgcn_sched_barrier(0);
     rec[0] = load_rec<kPolicy>(wt, wblock(b0), o16, o8, o2, o1, 0);
     dh = __builtin_amdgcn_raw_buffer_load_b16(wt, od + kTileD, wblock(b0), kPolicy);
@@ -319,7 +331,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
         if constexpr (kDecode)
             asm volatile("" : "+v"(nxt.hi), "+v"(nxt.lo));
         if constexpr (S == 0) {
-            dcur = half_bits_to_float(dh);
+            dcur = KG == 1 || b < b1 ? half_bits_to_float(dh) : 0.0f;
             asm volatile("" : "+v"(dcur));
         }
         if constexpr (S == 0 && !kLast) {
@@ -351,12 +363,12 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
         __syncthreads();                                                                                           \
     } while (0)
     int b = b0;
-    for (; b + 1 < b1; ++b) {
+    for (; b + 1 < end; ++b) {
         MAMBO_WIDE_BLOCK(0, 1);
         ++b;
         MAMBO_WIDE_BLOCK(1, 0);
     }
-    if (b < b1) {
+    if (b < end) {
         MAMBO_WIDE_STEPS(0, true);
     }
 #undef MAMBO_WIDE_BLOCK
@@ -366,6 +378,28 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
     for (int mt = MT / 2; mt < MT; ++mt) // the last block's sums that no step 0 followed
         scale_acc(mt, 0, 16);
+    if constexpr (KG == 2) {
+        // the second K group's sums over the first buffer (every wave has left it), added by the first
+        static_assert(W * MT * 4096 <= KG * kRows * 256, "one buffer holds a group's sums");
+        float4 *red = reinterpret_cast<float4 *>(s_vals0) + wave * (MT * 4 * 64) + lane;
+        __syncthreads();
+        if (kg)
+#pragma unroll
+            for (int j = 0; j < 4 * MT; ++j)
+                red[64 * j] = make_float4(acc[j / 4][4 * (j & 3)], acc[j / 4][4 * (j & 3) + 1],
+                                          acc[j / 4][4 * (j & 3) + 2], acc[j / 4][4 * (j & 3) + 3]);
+        __syncthreads();
+        if (kg)
+            return;
+#pragma unroll
+        for (int j = 0; j < 4 * MT; ++j) {
+            const float4 v = red[64 * j];
+            acc[j / 4][4 * (j & 3)] += v.x;
+            acc[j / 4][4 * (j & 3) + 1] += v.y;
+            acc[j / 4][4 * (j & 3) + 2] += v.z;
+            acc[j / 4][4 * (j & 3) + 3] += v.w;
+        }
+    }
     if (n < N) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -385,28 +419,34 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // The kernel's shapes, with what one workgroup of K blocks takes on a CU that holds 1, 2, ..
-// of them (as many as its registers allow): microseconds per launch round and per block.
+// of them (as many as its registers allow): microseconds per launch round and per block of a
+// K group.
 struct WideShape {
-    int mt, waves, resident;
+    int mt, waves, kg, resident;
     double round, block[3];
 };
-constexpr WideShape kWideShapes[] = {
-    {2, 4, 3, 0.37, {1.26, 1.82, 2.49}}, {4, 4, 2, 2.2, {1.64, 2.60, 0.0}}, {4, 8, 1, 1.35, {2.45, 0.0, 0.0}}};
+constexpr WideShape kWideShapes[] = {{2, 4, 1, 3, 0.37, {1.26, 1.82, 2.49}},
+                                     {2, 4, 2, 1, 1.6, {1.82, 0.0, 0.0}},
+                                     {4, 4, 1, 2, 2.2, {1.64, 2.60, 0.0}},
+                                     {4, 4, 2, 1, 2.7, {2.43, 0.0, 0.0}},
+                                     {4, 8, 1, 1, 1.35, {2.45, 0.0, 0.0}}};
 constexpr int kWideSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
 constexpr int64_t kCUs = 256;
 
 // Microseconds of a launch of `wgs` workgroups of `b` K blocks each writing `mb` MB of outputs,
 // K in `splits` slices: the busiest CU's rounds, the output stores, and with several slices
-// the zero fill and the f32 atomics (~1.5 TB/s). Fitted to 12000 launches (42 shapes of 128 to
-// 57344 rows, K 512 to 28672, 33 to 4096 tokens, each at every shape and split; rms error 6%);
-// the plan it picks is 1.2% behind the fastest measured one on average.
+// the zero fill and the f32 atomics (~1.5 TB/s alone). One K group fitted to 12000 launches (42
+// shapes of 128 to 57344 rows, K 512 to 28672, 33 to 4096 tokens, each at every shape and split;
+// rms error 6%), two to 250; the plan it picks is 1% behind the fastest measured one on average
+// over 66 shapes and token counts (most: 8%, 8192 x 4096 at 64 tokens).
 double wide_time(const WideShape &w, int64_t wgs, int64_t b, int splits, double mb)
 {
+    b = cdiv(b, w.kg);
     const int64_t per = cdiv(wgs, kCUs), full = per / w.resident, rem = per % w.resident;
     double t = 3.62 + w.round * (double)(full + (rem ? 1 : 0)) +
                (double)b * ((double)full * w.block[w.resident - 1] + (rem ? w.block[rem - 1] : 0.0)) + 0.25 * mb;
     if (splits > 1)
-        t += 1.48 + 0.67 * mb * splits;
+        t += 1.48 + 0.8 * mb * splits;
     return t;
 }
 
@@ -418,15 +458,15 @@ int64_t wide_workgroups(const mambo_projection *proj, int count, int waves)
     return wgs;
 }
 
-template <int MT, int W>
+template <int MT, int W, int KG>
 void launch_wide(const WidePlan &p, dim3 grid, hipStream_t stream, const uint8_t *xv, int64_t ldxv, const uint8_t *xs,
                  int64_t ldxs, int64_t m, const GroupArgs &ga, int blocks)
 {
     if (grid.y == 1)
-        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, kStreamPolicy>), grid, dim3(W * 64), 0, stream, xv, ldxv, xs, ldxs, m, ga,
+        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, KG, kStreamPolicy>), grid, dim3(W * KG * 64), 0, stream, xv, ldxv, xs, ldxs, m, ga,
                      blocks, p.bps, p.splits > 1);
     else
-        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, 0>), grid, dim3(W * 64), 0, stream, xv, ldxv, xs, ldxs, m, ga, blocks,
+        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, KG, 0>), grid, dim3(W * KG * 64), 0, stream, xv, ldxv, xs, ldxs, m, ga, blocks,
                      p.bps, p.splits > 1);
 }
 
@@ -448,15 +488,16 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
     // that were in a fixed order stay so; against an unsplit tiled plan from 9 K blocks on
     // (4-35%; on 4 and 8 blocks launches of 7-17 us, the 64-token tiles are 1-12% ahead) or
     // where 128 x 128 tiles give every CU one; against the dense kernel (which decodes a weight
-    // once per 32 tokens) where 64 x 128 tiles nearly fill the chip (57344 x 8192 at 48 tokens
-    // 133 against 77 us; at half a chip, 14336 x 8192, 37 against 46), or where its waves do
-    // not divide few K blocks (6204 x 2816 at 40 tokens 24 against 18).
+    // once per 32 tokens) where 64 x 128 tiles take 80 CUs (us at 40 tokens: 28672
+    // x 4096 46 against 25, 14336 x 8192 43 and 36, 10240 x 4096 21.3 and 20.1; 8192 x 4096,
+    // 64 workgroups, 16.3 and 19.9), or where its waves do not divide few K blocks and it takes 64
+    // rows a workgroup (6144 x 2816 23 against 16; with 32 rows, 4096 x 2816, 13.4 and 16.2).
     const bool split = blocks > cdiv(blocks, other.split_k);
     const int64_t row_wgs = wide_workgroups(proj, count, 4);
     const bool fills = row_wgs * cdiv(m, 128) >= kCUs;
     if (!split) {
         const int64_t wgs64 = row_wgs * cdiv(m, 64);
-        if (other.kernel == MAMBO_GEMM_DENSE ? !(wgs64 >= 192 || (blocks % 4 != 0 && blocks <= 11 && wgs64 >= 32))
+        if (other.kernel == MAMBO_GEMM_DENSE ? !(wgs64 >= 80 || (blocks % 4 != 0 && blocks <= 11 && other.tile_n >= 64))
                                              : !(blocks >= 9 || fills))
             return false;
     }
@@ -475,10 +516,14 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
             const int splits = (int)cdiv(blocks, bps);
             if (s > 1 && (!split || wgs * s > 1100 || blocks < 2 * s))
                 continue;
+            // two K groups only while every CU has at most one workgroup: beyond, other workgroups
+            // fill the waits (28672 x 4096 at 1024 tokens 207 us with one group, 230 with two)
+            if (w.kg > 1 && wgs * splits > kCUs)
+                continue;
             const double t = wide_time(w, wgs * splits, bps, splits, mb);
             if (best == 0.0 || t < best) {
                 best = t;
-                *plan = {w.mt, w.waves, splits, (int)bps};
+                *plan = {w.mt, w.waves, w.kg, splits, (int)bps};
             }
         }
     }
@@ -500,11 +545,15 @@ int mambo_wide_launch(const WidePlan &p, const uint8_t *xv, int64_t ldxv, const 
         wgs += cdiv(cdiv(proj[g].n, 32), p.waves);
     }
     const dim3 grid((unsigned)wgs, (unsigned)cdiv(m, 32 * p.mt), (unsigned)p.splits);
-    if (p.mt == 2)
-        launch_wide<2, 4>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
-    else if (p.waves == 4)
-        launch_wide<4, 4>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
+    if (p.mt == 2 && p.kg == 2)
+        launch_wide<2, 4, 2>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
+    else if (p.mt == 4 && p.kg == 2)
+        launch_wide<4, 4, 2>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
+    else if (p.mt == 4 && p.waves == 4)
+        launch_wide<4, 4, 1>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
+    else if (p.mt == 2)
+        launch_wide<2, 4, 1>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
     else
-        launch_wide<4, 8>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
+        launch_wide<4, 8, 1>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
     return mambo_check_launch("iq3s_fp8_matmul (wide)");
 }

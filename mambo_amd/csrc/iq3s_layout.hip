@@ -271,60 +271,74 @@ __global__ __launch_bounds__(256) void pack_fields_kernel(SoaSrc src, int64_t n,
         pack_lane(FieldBlock{src, b * n + row, row < n}, lane, packed + (t * blocks + b) * (int64_t)kTileBytes);
 }
 
-// 32 rows x kBlocks blocks per workgroup, one weight group (32 values) per thread and block: of a
-// block the workgroup reads contiguous runs of the fields (2 KiB of qs) and writes 32 whole
-// 256-byte pieces, where a thread per group along a row read 64 bytes of qs here and there.
-// Memory-bound (110 bytes in, 288 out per block), so all loads of the blocks come first.
-// 4096 x 14336: 25 -> 17.6 us, 28672 x 4096: 38.5 -> 31.5 us (5.8 TB/s; a copy moves 4.8), level
-// below 1024 x 8192. Nontemporal stores are slower (63 us at 28672 x 4096).
-constexpr int kDequantRows = 32;
-template <int kBlocks>
+// 32 rows x 4 blocks per workgroup, 16 values (half a weight group) per thread, row and block.
+// Memory-bound (110 bytes in, 288 out per block), so what counts is whole lines: a store of the
+// wave covers 1 KiB of values without holes (a thread with the 32 values of a group stored every
+// second 16 bytes, twice), the scales of a row leave in one piece of 128 bytes, and a
+// field of a block is read in runs of 32 rows (2 KiB of qs). With whole lines the nontemporal
+// hint pays: nothing written is read here again. Workgroups next to each other take blocks of the same rows.
+// Thread per group -> halves -> halves, nontemporal (us): 4096 x 14336 30.7 -> 22.2 -> 15.2 (7.4 TB/s; a
+// copy moves 4.8), 28672 x 4096 57 -> 40 -> 28, 8192 x 28672 107 -> 79 -> 54, 4096 x 4096 7.2 -> 6.4 ->
+// 5.8, 1024 x 4096 4.2 -> 4.2 -> 4.1. Rows before blocks in the launch 1-6% slower at 4096 columns, 16 x 8 the same,
+// 64 x 4 up to 25% slower.
+constexpr int kDequantRows = 32, kDequantBlocks = 4;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+
 __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict__ d, const uint32_t *__restrict__ qs,
                                                       const uint16_t *__restrict__ qh,
                                                       const int32_t *__restrict__ signs,
-                                                      const uint32_t *__restrict__ scales, int64_t n,
-                                                      int64_t blocks, uint8_t *__restrict__ values,
+                                                      const uint32_t *__restrict__ scales, int64_t n, int64_t blocks,
+                                                      uint32_t groups, uint8_t *__restrict__ values,
                                                       float *__restrict__ out_scales)
 {
     __shared__ uint32_t lut[512];
-    for (int i = threadIdx.x; i < 512; i += blockDim.x)
+    constexpr int kPasses = kDequantRows / 16;
+    static_assert(kDequantRows * kDequantBlocks * 2 == 256, "a thread writes four scales");
+    const int tid = threadIdx.x, u = tid & 15; // u: half of a group of the thread's row
+    for (int i = tid; i < 512; i += 256)
         lut[i] = c_grid.fp8[i];
-    __syncthreads();
-    const int g = (int)threadIdx.x & 7;
-    const int64_t row = (int64_t)blockIdx.x * kDequantRows + (threadIdx.x >> 3);
-    if (row >= n)
-        return;
-    for (int64_t b0 = (int64_t)blockIdx.y * kBlocks; b0 < blocks; b0 += (int64_t)gridDim.y * kBlocks) {
-        uint2 q[kBlocks];
-        uint32_t hb[kBlocks], sw[kBlocks], sc[kBlocks];
-        uint16_t db[kBlocks];
+    const int64_t row0 = (int64_t)(blockIdx.x / groups) * kDequantRows;
+    const int64_t b0 = (int64_t)(blockIdx.x % groups) * kDequantBlocks;
+    // all loads first; past the weight the last block and row again
+    const auto element = [&](int row, int j) { return min(b0 + j, blocks - 1) * n + min(row0 + row, n - 1); };
+    uint32_t q[kPasses][kDequantBlocks], hb[kPasses][kDequantBlocks], sw[kPasses][kDequantBlocks];
 #pragma unroll
-        for (int j = 0; j < kBlocks; ++j) { // all loads first; past the weight the last block again
-            const int64_t e = min(b0 + j, blocks - 1) * n + row;
-            q[j] = make_uint2(qs[e * 16 + 2 * g], qs[e * 16 + 2 * g + 1]);
-            hb[j] = reinterpret_cast<const uint8_t *>(qh)[e * 8 + g];
-            sw[j] = (uint32_t)signs[e * 8 + g];
-            sc[j] = scales[e];
-            db[j] = d[e];
+    for (int p = 0; p < kPasses; ++p)
+#pragma unroll
+        for (int j = 0; j < kDequantBlocks; ++j) {
+            const int64_t e = element(16 * p + (tid >> 4), j);
+            q[p][j] = qs[e * 16 + u];
+            hb[p][j] = (uint32_t)reinterpret_cast<const uint8_t *>(qh)[e * 8 + (u >> 1)] >> (4 * (u & 1));
+            sw[p][j] = reinterpret_cast<const uint16_t *>(signs)[e * 16 + u];
         }
+    // scales: row tid >> 3, half tid & 1 of its block (tid >> 1) & 3
+    const int64_t es = element(tid >> 3, (tid >> 1) & 3);
+    const uint32_t sc = scales[es] >> (16 * (tid & 1));
+    const float df = half_bits_to_float(d[es]);
+    __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kBlocks; ++j) {
-            const int64_t b = b0 + j;
-            if (b >= blocks)
-                break;
-            uint32_t out[8];
+    for (int p = 0; p < kPasses; ++p)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const uint32_t idx = (((c < 4 ? q[j].x : q[j].y) >> (8 * (c & 3))) & 0xFFu) | (((hb[j] >> c) & 1u) << 8);
-                const uint32_t nib = (sw[j] >> (4 * c)) & 15u;
+        for (int j = 0; j < kDequantBlocks; ++j) {
+            u32x4 out;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint32_t idx = ((q[p][j] >> (8 * c)) & 0xFFu) | (((hb[p][j] >> c) & 1u) << 8);
+                const uint32_t nib = (sw[p][j] >> (4 * c)) & 15u;
                 out[c] = lut[idx] | ((nib * 0x00204081u & 0x01010101u) << 7);
             }
-            uint4 *vp = reinterpret_cast<uint4 *>(values + (row * blocks + b) * 256 + 32 * g);
-            vp[0] = make_uint4(out[0], out[1], out[2], out[3]);
-            vp[1] = make_uint4(out[4], out[5], out[6], out[7]);
-            out_scales[(row * blocks + b) * 8 + g] =
-                half_bits_to_float(db[j]) * (float)(1u + 2u * ((sc[j] >> (4 * g)) & 15u));
+            const int64_t row = row0 + 16 * p + (tid >> 4), b = b0 + j;
+            if (row < n && b < blocks)
+                __builtin_nontemporal_store(out, reinterpret_cast<u32x4 *>(values + (row * blocks + b) * 256) + u);
         }
+    const int64_t row = row0 + (tid >> 3), b = b0 + ((tid >> 1) & 3);
+    if (row < n && b < blocks) {
+        f32x4 out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            out[i] = df * (float)(1u + 2u * ((sc >> (4 * i)) & 15u));
+        *reinterpret_cast<f32x4 *>(out_scales + (row * blocks + b) * 8 + 4 * (tid & 1)) = out;
     }
 }
 
@@ -389,15 +403,9 @@ extern "C" int mambo_iq3s_dequant(const uint16_t *d, const uint32_t *qs, const u
     MAMBO_REQUIRE(d && qs && qh && signs && scales && values && out_scales, MAMBO_ERR_VALUE, "null pointer");
     MAMBO_REQUIRE(n >= 1 && blocks >= 1, MAMBO_ERR_VALUE, "IQ3_S weight must have positive N and K");
     MAMBO_REQUIRE((uintptr_t)values % 16 == 0, MAMBO_ERR_VALUE, "values must be 16-byte aligned");
-    const int64_t total = n * blocks * 8;
-    MAMBO_REQUIRE((total + 255) / 256 <= 0x7FFFFFFF, MAMBO_ERR_VALUE, "weight too large");
-    // a single block per workgroup where four would leave CUs idle (1024 x 4096: 4.4 us with four,
-    // 3.7 with one; 4096 x 4096, 512 workgroups: 7.3 and 7.9; level from 6144 x 8192 on)
-    const int64_t rows = (n + kDequantRows - 1) / kDequantRows;
-    const bool four = rows * ((blocks + 3) / 4) >= 512;
-    const int64_t groups = four ? (blocks + 3) / 4 : blocks;
-    const dim3 grid((unsigned)rows, (unsigned)(groups < 65535 ? groups : 65535));
-    MAMBO_LAUNCH(four ? dequant_kernel<4> : dequant_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, d, qs, qh, signs, scales, n, blocks, values,
-                 out_scales);
+    const int64_t rows = (n + kDequantRows - 1) / kDequantRows, groups = (blocks + kDequantBlocks - 1) / kDequantBlocks;
+    MAMBO_REQUIRE(rows <= 0x7FFFFFFF / groups, MAMBO_ERR_VALUE, "weight too large");
+    MAMBO_LAUNCH(dequant_kernel, dim3((unsigned)(rows * groups)), dim3(256), 0, (hipStream_t)stream, d, qs, qh, signs,
+                 scales, n, blocks, (uint32_t)groups, values, out_scales);
     return mambo_check_launch("iq3s_dequant");
 }

@@ -1,5 +1,5 @@
 """Weight preparation and decoding at the edges of their workgroups (64 rows x 4 blocks or a tile;
-32 rows x 1 or 4 blocks), from every form of source: whole fields against numpy, bit for bit,
+32 rows x 4 blocks), from every form of source: whole fields against numpy, bit for bit,
 and the tile layout against the one that the byte path builds."""
 
 from __future__ import annotations
@@ -86,3 +86,25 @@ def test_prepare_of_repeated_rows(gpu):
     a = prepare_iq3_s_fields(x.expand(7000, -1, -1), pack=True)
     b = prepare_iq3_s_fields(x.expand(7000, -1, -1).contiguous(), pack=True)
     assert torch.equal(a.packed, b.packed) and torch.equal(a.signs, b.signs) and torch.equal(a.d, b.d)
+
+
+@pytest.mark.parametrize("n,blocks", [(1, 1), (31, 3), (33, 4), (64, 5), (100, 9)])
+def test_dequant_into_scales_of_any_float_alignment(gpu, n, blocks):
+    """Edges of the decoder's 32 rows x 4 blocks, the scales four bytes off a 16-byte boundary, and
+    nothing written outside either output."""
+    from mambo_amd import _native
+    from mambo_amd.utils.iq3_s_weight import prepare_iq3_s_fields
+    raw = make_synthetic_iq3_s(n, blocks * 256, seed=3 * n + blocks)
+    f = prepare_iq3_s_fields(torch.from_numpy(raw).to(gpu))
+    bits = torch.full((n * blocks * 256 + 64,), 0x5A, dtype=torch.uint8, device=gpu)
+    scales = torch.full((n * blocks * 8 + 2,), 12345.0, device=gpu)
+    step(f"dequant, scales off alignment [{n},{blocks},110]")
+    _native.check(_native.lib().mambo_iq3s_dequant(
+        f.d.data_ptr(), f.qs.data_ptr(), f.qh.data_ptr(), f.signs.data_ptr(), f.scales.data_ptr(), n, blocks,
+        bits[32:].data_ptr(), scales[1:].data_ptr(), _native.stream_handle(None)))
+    torch.cuda.synchronize()
+    want_bits, want_scales = oracle.dequant_iq3s_fp8(raw)
+    np.testing.assert_array_equal(bits[32:-32].cpu().numpy(), want_bits.ravel())
+    np.testing.assert_array_equal(scales[1:-1].cpu().numpy(), want_scales.ravel())
+    assert bool((bits[:32] == 0x5A).all()) and bool((bits[-32:] == 0x5A).all())
+    assert float(scales[0]) == 12345.0 and float(scales[-1]) == 12345.0

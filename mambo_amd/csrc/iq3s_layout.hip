@@ -17,6 +17,17 @@ namespace {
 
 __constant__ GridTables c_grid = kGridTables;
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Stores past the caches, for whole lines that nothing here reads again.
+template <class T>
+__device__ __forceinline__ void put(T v, void *p)
+{
+    __builtin_nontemporal_store(v, reinterpret_cast<T *>(p));
+}
+
 struct RawSrc {
     const uint8_t *raw;
     int64_t sn, sb, sbyte;
@@ -89,10 +100,9 @@ __device__ __forceinline__ void pack_lane(const Src &src, int l, uint8_t *__rest
         }
     // four 36-bit pieces to 144 bits
     const uint64_t lo = idx[0] | (idx[1] << 36), hi = (idx[1] >> 28) | (idx[2] << 8) | (idx[3] << 44);
-    *reinterpret_cast<uint4 *>(tile + kTileIdxA + 16 * l) =
-        make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    put(u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)}, tile + kTileIdxA + 16 * l);
     *reinterpret_cast<uint16_t *>(tile + kTileIdxB + 2 * l) = (uint16_t)(idx[3] >> 20);
-    *reinterpret_cast<uint2 *>(tile + kTileSigns + 8 * l) = make_uint2(sign[0], sign[1]);
+    put(u32x2{sign[0], sign[1]}, tile + kTileSigns + 8 * l);
     tile[kTileScales + l] = src.scale_byte(q);
     if (q == 0)
         *reinterpret_cast<uint16_t *>(tile + kTileD + 2 * r) = src.d_bits();
@@ -150,8 +160,11 @@ __global__ __launch_bounds__(256) void prepare_kernel(RawSrc src, int64_t n, int
 // workgroups per CU hide: 64 rows so that d and scales are stored in lines of 128 and 256 bytes
 // (a tile per workgroup wrote 32 and 64 of them, from different XCDs), four blocks so that the
 // lines which neighbouring segments share are a fourth of all. 28672 x 4096, fields and tiles:
-// 106 us a tile per workgroup -> 40 us (3.8 TB/s; a copy moves 4.8); two blocks 56, one 80, 96
-// registers for a fifth workgroup per CU (13 spilled) 46. 4096 x 14336: 45 -> 17 us.
+// 106 us a tile per workgroup -> 44 us, two blocks 56, one 80, 96 registers for a fifth workgroup per
+// CU (13 spilled) 46. The fields and a tile's index words and signs are stored nontemporal (nothing
+// here reads them again): 28672 x 4096 44 -> 29 us (5.3 TB/s; a copy moves 4.8), 4096 x 14336 24 ->
+// 17, 8192 x 28672 87 -> 58; tiles alone 25.6 -> 23.7, 15.1 -> 14.5, 68 -> 48. With the tile's
+// small pieces (32 to 128 bytes) nontemporal too 28672 x 4096 takes 32.
 constexpr int kPrepRows = 64, kPrepBlocks = 4;
 constexpr int kPrepPitch = (kPrepBlocks * kIq3sBlockBytes + 7) / 8 * 2 + 1; // words; odd: rows in all banks
 
@@ -208,8 +221,8 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const uint8_t *__rest
                 const int r = tid >> 2, c = tid & 3;
                 if (row0 + r < n) {
                     const ImageBlock o = block(r, j);
-                    *reinterpret_cast<uint4 *>(out.qs + ((b0 + j) * n + row0 + r) * 16 + 4 * c) =
-                        make_uint4(o.word(2 + 16 * c), o.word(6 + 16 * c), o.word(10 + 16 * c), o.word(14 + 16 * c));
+                    put(u32x4{o.word(2 + 16 * c), o.word(6 + 16 * c), o.word(10 + 16 * c), o.word(14 + 16 * c)},
+                        out.qs + ((b0 + j) * n + row0 + r) * 16 + 4 * c);
                 }
             }
         if (out.signs)
@@ -217,19 +230,19 @@ __global__ __launch_bounds__(256) void prepare_rows_kernel(const uint8_t *__rest
                 const int r = (tid & 127) >> 1, c = tid & 1;
                 if (row0 + r < n) {
                     const ImageBlock o = block(r, j);
-                    *reinterpret_cast<uint4 *>(out.signs + ((b0 + j) * n + row0 + r) * 8 + 4 * c) =
-                        make_uint4(o.word(74 + 16 * c), o.word(78 + 16 * c), o.word(82 + 16 * c), o.word(86 + 16 * c));
+                    put(u32x4{o.word(74 + 16 * c), o.word(78 + 16 * c), o.word(82 + 16 * c), o.word(86 + 16 * c)},
+                        out.signs + ((b0 + j) * n + row0 + r) * 8 + 4 * c);
                 }
             }
         if (wave < nb && row0 + lane < n) { // one block of every row per wave
             const ImageBlock o = block(lane, wave);
             const int64_t e = (b0 + wave) * n + row0 + lane;
             if (out.qh)
-                *reinterpret_cast<uint2 *>(out.qh + e * 4) = make_uint2(o.word(66), o.word(70));
+                put(u32x2{o.word(66), o.word(70)}, out.qh + e * 4);
             if (out.scales)
-                out.scales[e] = o.half(106) | (o.half(108) << 16);
+                put(o.half(106) | (o.half(108) << 16), out.scales + e);
             if (out.d)
-                out.d[e] = o.d_bits();
+                put(o.d_bits(), out.d + e);
         }
         const int64_t t = row0 / kTileRows + wave; // one 16-row tile per wave
         if (out.packed && t * kTileRows < n)
@@ -282,8 +295,6 @@ __global__ __launch_bounds__(256) void pack_fields_kernel(SoaSrc src, int64_t n,
 // 5.8, 1024 x 4096 4.2 -> 4.2 -> 4.1. Rows before blocks in the launch 1-6% slower at 4096 columns, 16 x 8 the same,
 // 64 x 4 up to 25% slower.
 constexpr int kDequantRows = 32, kDequantBlocks = 4;
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 
 __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict__ d, const uint32_t *__restrict__ qs,
                                                       const uint16_t *__restrict__ qh,

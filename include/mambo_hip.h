@@ -245,9 +245,10 @@ int mambo_iq3s_matmul_quantize_grouped_noalloc(const void *x, int x_dtype, int64
                                                const mambo_gemm_config *cfg, mambo_stream_t stream);
 
 /* The configuration mambo_iq3s_fp8_matmul uses when cfg == NULL (or all zero), except where
- * it takes the 32 x 32 MFMA kernel instead: from 33 tokens, on the shapes where that is the
- * faster one (mambo_amd/csrc/iq3s_wide.hip). That kernel splits K only where this
- * configuration does, and is not one that a caller can name. */
+ * another is the faster one for the call's shape: from 5 tokens the tiled kernel's small tiles
+ * without a K split (mambo_amd/csrc/iq3s_gemm.hip, small_tiles), from 33 tokens the 32 x 32
+ * MFMA kernel (mambo_amd/csrc/iq3s_wide.hip), which splits K only where this configuration
+ * does and is not one that a caller can name. */
 int mambo_gemm_default_config(int64_t m, int64_t n, int64_t blocks, mambo_gemm_config *out);
 
 /* Validates cfg for the shape (MAMBO_OK or MAMBO_ERR_VALUE with a reason). */

@@ -1956,6 +1956,72 @@ int zero_outputs(const GroupArgs &ga, int64_t m, hipStream_t s)
     return mambo_check_launch("zero_rows");
 }
 
+// At least what a dense or unsplit tiled configuration takes (us; measured on the shapes of small_tiles):
+// a dense kernel that splits K 7 us with its zero fill and 1.5 us per 100 M multiply-adds; else the
+// chain of a wave's blocks (0.44 us each up to 16 tokens, 0.8 with 32 per workgroup, 1.25 in the tiled kernel's
+// 64 x 128 tiles) or the decodes of the dense kernel's 16 rows x 32 tokens (0.8 to 1.4 ns each).
+double config_time(const mambo_gemm_config &c, int64_t m, int64_t n, int64_t blocks)
+{
+    if (c.kernel == MAMBO_GEMM_TILED)
+        return 3.8 + 1.25 * (double)cdiv(blocks, c.split_k);
+    if (c.split_k > 1)
+        return 7.0 + 1.5e-8 * 256.0 * (double)m * (double)n * (double)blocks;
+    const double decodes = (double)cdiv(n, kTileRows) * (double)cdiv(m, 32) * (double)blocks;
+    return 3.4 + std::max((m > 16 ? 0.8 : 0.44) * (double)cdiv(blocks, c.waves), (m > 32 ? 1.4e-3 : 0.8e-3) * decodes);
+}
+
+// The tiled kernel's small tiles (16 or 32 tokens, 16 to 64 weight rows): eight waves that share the
+// K blocks of 1, 2 or 4 row tiles, no K split; for launches that larger tiles leave most of the chip out of,
+// and for K that the dense kernel's waves do not divide. Each workgroup of a CU adds to its time, a
+// round half filled costs half (fitted to 930 launches of 128 to 20000 rows, K 512 to 28672, 5 to 400
+// tokens: rms error 5-6%; the tile it picks is 0.3% behind the fastest of the six).
+//
+// True and the configuration where that is faster than what else takes the call, in other_us
+// microseconds (0: not known). Between 17 and 32 tokens the 32 x 64 tiles of that range stay. us
+// before and after: 4096 x 4096 at 48 / 128 tokens 11.6 -> 8.9, 17.4 -> 12.4; 1024 x 4096 10.5 -> 6.9 at
+// both; 2048 x 2816 at 128 16.8 -> 7.6; 4096 x 14336 at 48 27 -> 21; 8192 x 28672 at 48 73 -> 60; 640 x 3328
+// at 10 10.0 -> 5.5; 1314 x 18688 at 18 36 -> 15; geometric mean of 290 random shapes at 33 to 400 tokens 0.74.
+bool small_tiles(int64_t m, const mambo_projection *proj, int count, int64_t blocks, const uint8_t *xs, int64_t ldxs,
+                 const mambo_gemm_config &other, double other_us, mambo_gemm_config *out)
+{
+    struct Tile {
+        int tokens, rows, k_groups;
+        double launch, round, wait, block; // us: fixed, per workgroup of a CU, per block at least, per block and workgroup
+    };
+    static constexpr Tile kTiles[] = {{32, 16, 8, 2.48, 1.74, 0.186, 0.199}, {32, 32, 4, 3.34, 0.56, 0.298, 0.259},
+                                      {32, 64, 2, 3.22, 0.45, 0.521, 0.462}, {16, 16, 8, 2.89, 0.99, 0.144, 0.124},
+                                      {16, 32, 4, 2.99, 0.76, 0.242, 0.206}, {16, 64, 2, 3.13, 0.70, 0.411, 0.398}};
+    // (the scale rows are copied as dwords, as the tiled kernel asks)
+    if (m < 5 || m > 400 || blocks < 2 || (uintptr_t)xs % 8 != 0 || ldxs % 8 != 0 ||
+        (other.kernel == MAMBO_GEMM_TILED && m <= 32))
+        return false;
+    int64_t n = 0;
+    for (int g = 0; g < count; ++g)
+        n += proj[g].n;
+    const double mn = (double)m * (double)n;
+    double best = 0.97 * other_us;
+    bool found = false;
+    for (const Tile &t : kTiles) {
+        int64_t wgs = 0;
+        for (int g = 0; g < count; ++g)
+            wgs += cdiv(proj[g].n, t.rows) * cdiv(m, t.tokens);
+        const double per_cu = 0.5 * ((double)wgs / kCUs + (double)cdiv(wgs, kCUs));
+        const double us = t.launch + t.round * per_cu + 0.68e-6 * mn +
+                          (double)(cdiv(blocks, t.k_groups) * t.k_groups) * std::max(t.wait, t.block * per_cu);
+        if (us < best) {
+            best = us;
+            *out = {};
+            out->kernel = MAMBO_GEMM_TILED;
+            out->waves = 8;
+            out->split_k = 1;
+            out->tile_m = t.tokens;
+            out->tile_n = t.rows;
+            found = true;
+        }
+    }
+    return found;
+}
+
 // quant: -1 when xv/xs are MXFP8 activations; else xv holds unquantized rows of dtype
 // quant (ldxv in elements, xs unused) for the stream kernel to quantize itself, and the
 // call returns kNotFused, launching nothing, when the configuration cannot do that.
@@ -2013,17 +2079,30 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
         if (rc)
             return rc;
     }
-    // A call that leaves the configuration to the library takes the 32 x 32 MFMA kernel where
-    // that is the faster one.
-    WidePlan wide;
-    if (quant < 0 && (cfg == nullptr || all_default(*cfg)) &&
-        mambo_wide_plan(m, proj, count, blocks, ldxv, xs, ldxs, c, &wide)) {
-        if (wide.splits > 1) {
-            rc = zero_outputs(ga, m, s);
-            if (rc)
-                return rc;
+    // A call that leaves the configuration to the library takes the 32 x 32 MFMA kernel or small
+    // tiles where they are the faster ones.
+    if (quant < 0 && (cfg == nullptr || all_default(*cfg))) {
+        WidePlan wide;
+        bool have_wide = mambo_wide_plan(m, proj, count, blocks, ldxv, xs, ldxs, c, &wide);
+        double us = have_wide ? wide.us : 0.0;
+        // few rows and a long K: the dense kernel's K split (199 x 19712 at 47 tokens 10.5 and 12.7 us)
+        if (!have_wide || (c.kernel == MAMBO_GEMM_DENSE && c.split_k > 1)) {
+            const double base = config_time(c, m, n_total, blocks);
+            have_wide = have_wide && us <= 0.9 * base;
+            us = have_wide ? us : base;
         }
-        return mambo_wide_launch(wide, xv, ldxv, xs, ldxs, m, proj, count, blocks, s);
+        mambo_gemm_config small;
+        if (small_tiles(m, proj, count, blocks, xs, ldxs, c, us, &small) &&
+            mambo_gemm_check_config(m, n_total, blocks, &small) == MAMBO_OK) {
+            c = small;
+        } else if (have_wide) {
+            if (wide.splits > 1) {
+                rc = zero_outputs(ga, m, s);
+                if (rc)
+                    return rc;
+            }
+            return mambo_wide_launch(wide, xv, ldxv, xs, ldxs, m, proj, count, blocks, s);
+        }
     }
     if (quant >= 0) { // in-kernel quantization: stream kernel, one sub-tile, rows staged in LDS
         const int64_t esz = quant == MAMBO_DTYPE_BF16 ? 2 : 4;

@@ -9,6 +9,7 @@ struct WidePlan {
     int kg;     // K groups of waves per workgroup
     int splits; // K slices (more than one: f32 atomics into outputs zeroed beforehand)
     int bps;    // K blocks per slice
+    double us;  // what the plan's cost model expects of it
 };
 
 // Whether the kernel takes the call (it can, and is the faster choice), and its plan. other: the

@@ -32,6 +32,11 @@
 // each at its fastest split (us): 28672 x 4096 at 48 tokens 29 -> 25.6, 10240 x 8192 at 256
 // 59 -> 51, 6144 x 4096 at 256 25 -> 22, 8192 x 28672 at 128 80 -> 72, 4096 x 14336 at 256
 // 54 -> 43. Launches that fill the chip gain nothing from it (57344 x 8192 at 48: 82 and 85).
+// Four groups of two waves (64 x 64 tiles) where even that leaves CUs without a workgroup: 8192 x
+// 8192 at 96 and 128 tokens 29 -> 26 and 31 -> 27, 6144 x 4096 18 -> 15.5 and 19 -> 16.
+// One 32-token sub-tile (MT = 1, reads a K step ahead) was built too and is level with the tiled
+// and dense kernels at 8 to 32 tokens (57344 x 8192 at 16 / 32 63 and 70 us against 54 and 70, 28672
+// x 4096 18 and 20 against 17 and 20): left out.
 //
 // Measured against the kernels it takes over from, same box, one launch in a replayed graph
 // over rotated weights (us): 57344 x 8192 at 40 / 128 / 512 tokens 133 -> 77, 133 -> 109, 456 ->
@@ -108,16 +113,15 @@ __device__ __forceinline__ void fetch_words(const WState &st, const uint8_t *lvl
     }
 }
 // Codes C0 .. C0+N-1 of the step from their codebook words.
-template <int H, int C0, int N>
-__device__ __forceinline__ void finish_words(const WState &st, const uint32_t (&lw)[8], const uint4 (&tab)[2],
-                                             StepOps &o)
+template <int C0, int N>
+__device__ __forceinline__ void finish_words(uint32_t p, const uint32_t (&lw)[8], const uint4 (&tab)[2], StepOps &o)
 {
     if constexpr (N > 0) {
         int hi, lo;
-        split_word<C0>(lw[C0], st.p[H], tab[C0 / 4], hi, lo);
+        split_word<C0>(lw[C0], p, tab[C0 / 4], hi, lo);
         o.hi[C0] = hi;
         o.lo[C0] = lo;
-        finish_words<H, C0 + 1, N - 1>(st, lw, tab, o);
+        finish_words<C0 + 1, N - 1>(p, lw, tab, o);
     }
 }
 
@@ -131,7 +135,7 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
     constexpr int kRows = 32 * MT;
     constexpr int kVCopies = kRows / 4 / W;
     static_assert(MT % 2 == 0, "the scalings are split over two steps");
-    static_assert(kRows / 4 % W == 0 && MT <= W && 4 * W % 16 == 0, "staging must spread evenly over the waves");
+    static_assert(kRows / 4 % W == 0 && MT <= W && (W % 4 == 0 || 4 % W == 0), "staging must spread evenly over the waves");
     // the alignments place the tables and scales first, below the 64 KiB that an LDS
     // instruction's offset reaches (above it every read needs its address or-ed together: 38
     // more vector instructions per block, 3-5% of the kernel)
@@ -177,8 +181,14 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
     };
     const __amdgpu_buffer_rsrc_t xrows = rows_rsrc(xv, ldxv, B * 256), srows = rows_rsrc(xs, ldxs, B * 8);
     const int srow = wave & (MT - 1); // waves past MT repeat a scale copy (the same bytes): no branch
-    const uint32_t voff = (uint32_t)(4 * wave + (lane >> 4)) * (uint32_t)ldxv +
-                          16u * (uint32_t)((lane & 15) ^ ((4 * wave + (lane >> 4)) & 15));
+    // copy j covers rows 4 * (wave + W * j) .. + 3; with fewer than four waves the swizzle of a lane's
+    // chunk repeats every 4 / W copies
+    constexpr int kSwizzles = W < 4 ? 4 / W : 1;
+    uint32_t voff[kSwizzles];
+#pragma unroll
+    for (int j = 0; j < kSwizzles; ++j)
+        voff[j] = (uint32_t)(4 * wave + (lane >> 4)) * (uint32_t)ldxv +
+                  16u * (uint32_t)((lane & 15) ^ ((4 * (wave + W * j) + (lane >> 4)) & 15));
     const uint32_t soff_stage = (uint32_t)(32 * srow + (lane >> 1)) * (uint32_t)ldxs + 4u * (lane & 1);
 
     const uint32_t a0 = (uint32_t)(kg * kRows * 256) + 256u * r32 + 16u * (uint32_t)(g ^ col);
@@ -192,22 +202,26 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
         for (int i = 0; i < 16; ++i)
             acc[mt][i] = c[mt][i] = 0.0f;
-    // K group kg takes blocks [b0, end); those from b1 on count with a zero d
+    // K group kg takes blocks [b0, end); those from b1 on are a block again with its sums scaled to
+    // 2^-128 (an infinite sum must not meet the zero) and a zero d
     const int z0 = blockIdx.z * bps, b1 = min(B, z0 + bps), per = (b1 - z0 + KG - 1) / KG;
     const int b0 = z0 + kg * per, end = b0 + per;
     auto wblock = [&](int b) { return (uint32_t)min(b, b1 - 1) * kTileBytes; };
 
     auto stage = [&](uint8_t *vals, uint8_t *scl, int b) {
 #pragma unroll
-        for (int j = 0; j < kVCopies; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrows, (lds_ptr)(vals + kg * kRows * 256 + 1024 * (wave + W * j)), 16, voff,
-                                                     256u * b + (uint32_t)(4 * W * j) * (uint32_t)ldxv, 0, 0);
+        for (int j = 0; j < kVCopies; ++j) {
+            const uint32_t vo = voff[j % kSwizzles]; // (the host pass drops the kernel with the element as an argument)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrows, (lds_ptr)(vals + kg * kRows * 256 + 1024 * (wave + W * j)),
+                                                     16, vo, 256u * b + (uint32_t)(4 * W * j) * (uint32_t)ldxv, 0, 0);
+        }
         __builtin_amdgcn_raw_ptr_buffer_load_lds(srows, (lds_ptr)(scl + kg * kRows * 8 + 256 * srow), 4, soff_stage, 8u * b, 0, 0);
     };
 
     WRec rec[2];
     uint16_t dh;
     StepOps op[2];
+    int bscale = 128;
     float dcur = 0.0f;
     v8i a[2];
     int sc[2];
@@ -237,7 +251,7 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
         uint32_t lw[8];
         const uint4 tab[2] = {split_entry<0, 0>(s_split, st.sc), split_entry<0, 1>(s_split, st.sc)};
         fetch_words<0, 0, 8>(st, lvl, lw);
-        finish_words<0, 0, 8>(st, lw, tab, op[0]);
+        finish_words<0, 8>(st.p[0], lw, tab, op[0]);
     }
 
     // Activation fragment of sub-tile mt for K step S (= 2r + h): row r32, 16-byte chunks 8r + 2h +
@@ -292,10 +306,10 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
                         for (int i = 0; i < 16; ++i)
                             zero[i] = 0.0f;
                         c[mt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[sl], cur.hi, zero, 0, 0, h, sc[sl], 0,
-                                                                                128);
+                                                                                bscale);
                     } else {
                         c[mt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[sl], cur.hi, c[mt], 0, 0, h, sc[sl],
-                                                                                0, 128);
+                                                                                0, bscale);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (mt == 0 && kDecode) {
@@ -314,15 +328,15 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
                     if constexpr (due >= 0)
                         scale_acc(due, 0, 8);
                     if constexpr (mt > 0 && kDecode)
-                        finish_words<nh, d0, dn / 2>(st, lw, tab, nxt);
+                        finish_words<d0, dn / 2>(st.p[nh], lw, tab, nxt);
                     __builtin_amdgcn_sched_barrier(0);
                     c[mt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[sl], cur.lo, c[mt], 0, 0, h, sc[sl], 0,
-                                                                            128);
+                                                                            bscale);
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (due >= 0)
                         scale_acc(due, 8, 8);
                     if constexpr (mt > 0 && kDecode)
-                        finish_words<nh, d0 + dn / 2, dn - dn / 2>(st, lw, tab, nxt);
+                        finish_words<d0 + dn / 2, dn - dn / 2>(st.p[nh], lw, tab, nxt);
                     __builtin_amdgcn_sched_barrier(0);
                 }(),
                 ...);
@@ -351,6 +365,8 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
 #define MAMBO_WIDE_STEPS(CUR, LAST)                                                                                \
     load_frag.template operator()<0>(s_vals##CUR, s_scale##CUR, 0, 0);                                             \
     __builtin_amdgcn_sched_barrier(0);                                                                             \
+    if constexpr (KG > 1)                                                                                          \
+        bscale = b < b1 ? 128 : 0;                                                                                 \
     kstep.template operator()<0, LAST>(s_vals##CUR, s_scale##CUR, b);                                              \
     kstep.template operator()<1, LAST>(s_vals##CUR, s_scale##CUR, b);                                              \
     kstep.template operator()<2, LAST>(s_vals##CUR, s_scale##CUR, b);                                              \
@@ -378,27 +394,30 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
     for (int mt = MT / 2; mt < MT; ++mt) // the last block's sums that no step 0 followed
         scale_acc(mt, 0, 16);
-    if constexpr (KG == 2) {
-        // the second K group's sums over the first buffer (every wave has left it), added by the first
-        static_assert(W * MT * 4096 <= KG * kRows * 256, "one buffer holds a group's sums");
+    if constexpr (KG > 1) {
+        // the other K groups' sums over the first buffer (every wave has left it), added by the first
+        static_assert((KG - 1) * W * MT * 4096 <= KG * kRows * 256, "one buffer holds the groups' sums");
         float4 *red = reinterpret_cast<float4 *>(s_vals0) + wave * (MT * 4 * 64) + lane;
         __syncthreads();
         if (kg)
 #pragma unroll
             for (int j = 0; j < 4 * MT; ++j)
-                red[64 * j] = make_float4(acc[j / 4][4 * (j & 3)], acc[j / 4][4 * (j & 3) + 1],
-                                          acc[j / 4][4 * (j & 3) + 2], acc[j / 4][4 * (j & 3) + 3]);
+                red[(kg - 1) * (W * MT * 4 * 64) + 64 * j] =
+                    make_float4(acc[j / 4][4 * (j & 3)], acc[j / 4][4 * (j & 3) + 1], acc[j / 4][4 * (j & 3) + 2],
+                                acc[j / 4][4 * (j & 3) + 3]);
         __syncthreads();
         if (kg)
             return;
 #pragma unroll
-        for (int j = 0; j < 4 * MT; ++j) {
-            const float4 v = red[64 * j];
-            acc[j / 4][4 * (j & 3)] += v.x;
-            acc[j / 4][4 * (j & 3) + 1] += v.y;
-            acc[j / 4][4 * (j & 3) + 2] += v.z;
-            acc[j / 4][4 * (j & 3) + 3] += v.w;
-        }
+        for (int k = 0; k < KG - 1; ++k)
+#pragma unroll
+            for (int j = 0; j < 4 * MT; ++j) {
+                const float4 v = red[k * (W * MT * 4 * 64) + 64 * j];
+                acc[j / 4][4 * (j & 3)] += v.x;
+                acc[j / 4][4 * (j & 3) + 1] += v.y;
+                acc[j / 4][4 * (j & 3) + 2] += v.z;
+                acc[j / 4][4 * (j & 3) + 3] += v.w;
+            }
     }
     if (n < N) {
 #pragma unroll
@@ -428,6 +447,7 @@ struct WideShape {
 constexpr WideShape kWideShapes[] = {{2, 4, 1, 3, 0.37, {1.26, 1.82, 2.49}},
                                      {2, 4, 2, 1, 1.6, {1.82, 0.0, 0.0}},
                                      {4, 4, 1, 2, 2.2, {1.64, 2.60, 0.0}},
+                                     {2, 2, 4, 1, 1.6, {2.3, 0.0, 0.0}},
                                      {4, 4, 2, 1, 2.7, {2.43, 0.0, 0.0}},
                                      {4, 8, 1, 1, 1.35, {2.45, 0.0, 0.0}}};
 constexpr int kWideSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -462,12 +482,12 @@ template <int MT, int W, int KG>
 void launch_wide(const WidePlan &p, dim3 grid, hipStream_t stream, const uint8_t *xv, int64_t ldxv, const uint8_t *xs,
                  int64_t ldxs, int64_t m, const GroupArgs &ga, int blocks)
 {
-    if (grid.y == 1)
-        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, KG, kStreamPolicy>), grid, dim3(W * KG * 64), 0, stream, xv, ldxv, xs, ldxs, m, ga,
-                     blocks, p.bps, p.splits > 1);
+    if (grid.y > 1)
+        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, KG, 0>), grid, dim3(W * KG * 64), 0, stream, xv, ldxv, xs, ldxs, m,
+                     ga, blocks, p.bps, p.splits > 1);
     else
-        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, KG, 0>), grid, dim3(W * KG * 64), 0, stream, xv, ldxv, xs, ldxs, m, ga, blocks,
-                     p.bps, p.splits > 1);
+        MAMBO_LAUNCH((gemm_wide_kernel<MT, W, KG, kStreamPolicy>), grid, dim3(W * KG * 64), 0, stream, xv, ldxv, xs,
+                     ldxs, m, ga, blocks, p.bps, p.splits > 1);
 }
 
 } // namespace
@@ -523,7 +543,7 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
             const double t = wide_time(w, wgs * splits, bps, splits, mb);
             if (best == 0.0 || t < best) {
                 best = t;
-                *plan = {w.mt, w.waves, w.kg, splits, (int)bps};
+                *plan = {w.mt, w.waves, w.kg, splits, (int)bps, t};
             }
         }
     }
@@ -545,15 +565,16 @@ int mambo_wide_launch(const WidePlan &p, const uint8_t *xv, int64_t ldxv, const 
         wgs += cdiv(cdiv(proj[g].n, 32), p.waves);
     }
     const dim3 grid((unsigned)wgs, (unsigned)cdiv(m, 32 * p.mt), (unsigned)p.splits);
-    if (p.mt == 2 && p.kg == 2)
-        launch_wide<2, 4, 2>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
-    else if (p.mt == 4 && p.kg == 2)
-        launch_wide<4, 4, 2>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
-    else if (p.mt == 4 && p.waves == 4)
-        launch_wide<4, 4, 1>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
-    else if (p.mt == 2)
-        launch_wide<2, 4, 1>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
-    else
-        launch_wide<4, 8, 1>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks);
+    const auto is = [&](int mt, int waves, int kg) { return p.mt == mt && p.waves == waves && p.kg == kg; };
+#define MAMBO_WIDE_SHAPE(MT, W, KG)                                                                                \
+    if (is(MT, W, KG))                                                                                             \
+    launch_wide<MT, W, KG>(p, grid, stream, xv, ldxv, xs, ldxs, m, ga, (int)blocks)
+    MAMBO_WIDE_SHAPE(2, 2, 4);
+    MAMBO_WIDE_SHAPE(2, 4, 1);
+    MAMBO_WIDE_SHAPE(2, 4, 2);
+    MAMBO_WIDE_SHAPE(4, 4, 1);
+    MAMBO_WIDE_SHAPE(4, 4, 2);
+    MAMBO_WIDE_SHAPE(4, 8, 1);
+#undef MAMBO_WIDE_SHAPE
     return mambo_check_launch("iq3s_fp8_matmul (wide)");
 }

@@ -45,7 +45,9 @@ def project(gpu, xv, xs, raws, config=None, pad=0):
 SHAPES = [(257, [100], 9), (320, [33], 10), (256, [16, 17, 48], 11), (300, [130], 16), (385, [64, 1], 33),
           (1000, [4090], 4), (1025, [3000, 1100], 5), (961, [8190], 5), (1024, [8000, 190], 4),
           (33, [6204], 11), (63, [12288 + 16], 4), (40, [10200], 5), (128, [4100, 4000], 23), (129, [8192], 13),
-          (65, [1000], 64), (2048, [16000], 4), (48, [57344], 4)]
+          (65, [1000], 64), (2048, [16000], 4), (48, [57344], 4),
+          # four K groups of 64 x 64 tiles: blocks that leave one to three groups short
+          (96, [8100], 33), (128, [6000, 130], 18), (97, [8192], 15)]
 
 
 @pytest.mark.parametrize("m,ns,blocks", SHAPES)
@@ -87,6 +89,49 @@ def test_wide_scales_and_special_values(gpu, m, n, blocks):
         j = ok[i]
         if j.any():
             assert rel_l2(got[i, j], want[i, j]) < 1e-4
+
+
+# tokens, rows of each projection, K blocks for the small tiles that take launches of few
+# workgroups: each tile (16 and 32 tokens, 16, 32 and 64 rows), first and last tokens and rows of a tile, blocks
+# that divide among eight waves' K groups or leave some without, the last token count of the rule
+SMALL = [(33, [1], 4), (64, [16, 17], 5), (65, [100, 33, 1], 8), (48, [4090], 16), (96, [1000], 9), (129, [2050], 7),
+         (256, [700, 64], 13), (48, [8190], 23), (128, [4100], 4), (34, [3000], 112), (5, [640], 13), (16, [1, 300], 3),
+         (17, [250], 2), (12, [2300], 47), (400, [330], 7), (400, [3170], 2)]
+
+
+@pytest.mark.parametrize("m,ns,blocks", SMALL)
+def test_launches_of_few_workgroups(gpu, m, ns, blocks):
+    """Against the oracle, and the same bits again (no K split takes these calls)."""
+    k = 256 * blocks
+    raws = [make_synthetic_iq3_s(n, k, seed=11 * m + i) for i, n in enumerate(ns)]
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    xv, xs = oracle.quantize_mxfp8(x)
+    step(f"few workgroups M={m} N={ns} K={k}")
+    first = project(gpu, xv, xs, raws, pad=3)
+    for o, raw in zip(first, raws):
+        rows = np.unique(np.r_[np.arange(min(40, raw.shape[0])), np.arange(max(0, raw.shape[0] - 40), raw.shape[0])])
+        assert np.isfinite(o).all()
+        assert rel_l2(o[:, rows], oracle.iq3s_fp8_matmul(xv, xs, raw[rows], threads=oracle.default_threads())) < 1e-4
+    for o, again in zip(first, project(gpu, xv, xs, raws)):
+        assert np.array_equal(o, again)
+
+
+@pytest.mark.parametrize("m,n,blocks", [(128, 6000, 17), (300, 130, 9)])
+def test_wide_infinite_sums(gpu, m, n, blocks):
+    """A token whose sums overflow f32: infinities (no NaN from a K group's missing last block),
+    as the tiled kernel gives them, and finite values elsewhere."""
+    k = 256 * blocks
+    raw = make_synthetic_iq3_s(n, k, seed=n)
+    xv = np.full((m, k), 0x38, dtype=np.uint8)  # 1.0
+    xs = np.full((m, k // 32), 127, dtype=np.uint8)
+    xv[7], xs[7] = 0x7E, 254  # 448 * 2^127
+    step(f"wide infinities M={m} N={n} K={k}")
+    got, = project(gpu, xv, xs, [raw])
+    want, = project(gpu, xv, xs, [raw], config={"kernel": 2, "tile_m": 64, "tile_n": 128, "waves": 8, "split_k": 1})
+    assert np.isfinite(np.delete(got, 7, 0)).all() and not np.isfinite(want[7]).any()
+    assert np.array_equal(np.isinf(got[7]).any(), np.isinf(want[7]).any())
+    last = blocks - 1
+    assert last % 2 == 0  # both counts leave a group's last block out
 
 
 def test_wide_same_bits_without_a_split_and_under_capture(gpu):

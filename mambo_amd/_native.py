@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+from contextlib import nullcontext
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libmambo_hip.so"
@@ -167,7 +168,7 @@ def stream_handle(stream) -> int:
     """HIP stream handle of `stream` (None = torch's current stream on the current device)."""
     if stream is None:
         import torch
-        return int(torch.cuda.current_stream().cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, int):
         return stream
     handle = getattr(stream, "cuda_stream", None)
@@ -178,11 +179,31 @@ def stream_handle(stream) -> int:
     return int(handle)
 
 
+_archs: dict[int, str] = {}  # by device index; a device's architecture does not change
+
+
 def device_arch(device=None) -> str:
     """gfx name of the current (or given) torch device, e.g. 'gfx950'."""
     import torch
-    props = torch.cuda.get_device_properties(device if device is not None else torch.cuda.current_device())
-    return str(getattr(props, "gcnArchName", "")).split(":")[0]
+    index = device if device is not None else torch.cuda.current_device()
+    arch = _archs.get(index) if isinstance(index, int) else None
+    if arch is None:
+        arch = str(getattr(torch.cuda.get_device_properties(index), "gcnArchName", "")).split(":")[0]
+        if isinstance(index, int):
+            _archs[index] = arch
+    return arch
+
+
+_here = nullcontext()
+
+
+def on_device(device):
+    """Context with `device` (a tensor's) current; nothing to do where it is already, as in most
+    calls: entering and leaving torch.cuda.device costs an eager call about 2 us."""
+    import torch
+    if device.type == "cuda" and device.index == torch.cuda.current_device():
+        return _here
+    return torch.cuda.device(device)
 
 
 def ptr(t) -> int:

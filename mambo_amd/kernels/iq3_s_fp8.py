@@ -132,7 +132,7 @@ def launch_dequant_iq3_s(iq3_weight: IQ3SFields, *, tile_n: int = 1, stream=None
     dev = iq3_weight.d.device
     values = torch.empty((n_rows, blocks * 256), dtype=torch.uint8, device=dev)
     scales = torch.empty((n_rows, blocks * 8), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         _native.check(_native.lib().mambo_iq3s_dequant(*(t.data_ptr() for t in fields), n_rows, blocks,
                                                        values.data_ptr(), scales.data_ptr(),
                                                        _native.stream_handle(stream)), "launch_dequant_iq3_s")
@@ -204,7 +204,7 @@ def launch_iq3_s_fp8_matmul(x_values: torch.Tensor, x_scales: torch.Tensor, iq3_
     k = k_blocks * IQ3_S_BLOCK_VALUES
     x_values, x_scales, m = _prepare_activations(x_values, x_scales, k)
     dev = x_values.device
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         cfg = _native.GemmConfig.from_dict(config if config is not None else select_config(m, n_rows, k))
         packed = ensure_packed(iq3_weight, stream)
         out = _output(out, m, n_rows, dev)
@@ -239,7 +239,7 @@ def launch_iq3_s_fp8_matmul_grouped(x_values: torch.Tensor, x_scales: torch.Tens
     if outs is not None and len(outs) != len(weights):
         raise ValueError("outs must hold one output per weight")
     n_total = sum(n for n, _ in dims)
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         cfg = _native.GemmConfig.from_dict(config if config is not None else select_config(m, n_total, k))
         result = [_output(None if outs is None else outs[i], m, n, dev) for i, (n, _) in enumerate(dims)]
         projections = (_native.Projection * len(weights))()
@@ -283,7 +283,7 @@ def launch_iq3_s_matmul_quantize(x: torch.Tensor, iq3_weights, *, stream=None, c
     if outs is not None and len(outs) != len(weights):
         raise ValueError("outs must hold one output per weight")
     n_total = sum(n for n, _ in dims)
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         cfg = _native.GemmConfig.from_dict(config if config is not None else select_config(m, n_total, k))
         result = [_output(None if outs is None else outs[i], m, n, dev) for i, (n, _) in enumerate(dims)]
         projections = (_native.Projection * len(weights))()
@@ -324,7 +324,7 @@ def new_chain_sync(device=None) -> torch.Tensor:
 def chain_status(sync: torch.Tensor) -> None:
     """Raise RuntimeError if a chained call on ``sync`` had a dependency wait time out
     (synchronises with the device; clears the reported status)."""
-    with torch.cuda.device(sync.device):
+    with _native.on_device(sync.device):
         _native.check(_native.lib().mambo_chain_status(sync.data_ptr()), "chain_status")
 
 
@@ -380,7 +380,7 @@ def launch_iq3_s_fp8_matmul_chain(launches, *, stream=None, waves: int = 0, sync
             raise ValueError(f"launch {i}: x must be uint8 (MXFP8), float32 or bfloat16, got {x.dtype}")
         if cl.outs is not None and len(cl.outs) != len(weights):
             raise ValueError(f"launch {i}: outs must hold one output per weight")
-        with torch.cuda.device(dev):
+        with _native.on_device(dev):
             outs = [_output(None if cl.outs is None else cl.outs[j], m, n, dev) for j, (n, _) in enumerate(dims)]
             for j, (w, (n, _)) in enumerate(zip(weights, dims)):
                 desc.proj[j] = _native.Projection(ensure_packed(w, stream).data_ptr(), n, outs[j].data_ptr(),
@@ -390,7 +390,7 @@ def launch_iq3_s_fp8_matmul_chain(launches, *, stream=None, waves: int = 0, sync
     cfg = _native.ChainConfig()
     cfg.waves, cfg.tiles_per_workgroup, cfg.timeout_us, cfg.wait_bias = waves, tiles_per_workgroup, timeout_us, \
         wait_bias
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         if sync is None:
             sync = new_chain_sync(dev)
         if sync.dtype not in (torch.int32, torch.uint32) or sync.numel() < _native.CHAIN_SYNC_WORDS \

@@ -55,7 +55,7 @@ def launch_quantize_fp8(x: torch.Tensor, *, tile_m: int | None = None, tile_k_gr
     if not x.is_cuda:
         raise ValueError("activation must be a GPU tensor")
     if tile_m is None or tile_k_groups is None:
-        with torch.cuda.device(x.device):
+        with _native.on_device(x.device):
             config = _activation_config(x.shape[0])
         tile_m = config["tile_m"] if tile_m is None else tile_m
         tile_k_groups = config["tile_k_groups"] if tile_k_groups is None else tile_k_groups
@@ -73,7 +73,7 @@ def launch_quantize_fp8(x: torch.Tensor, *, tile_m: int | None = None, tile_k_gr
                 or scales.shape != (m, k // 32) or scales.dtype != torch.uint8 or scales.stride(1) != 1:
             raise ValueError("out must be (uint8 [M,K], uint8 [M,K/32]) with unit column stride")
     dtype = _native.DTYPE_F32 if x.dtype == torch.float32 else _native.DTYPE_BF16
-    with torch.cuda.device(x.device):
+    with _native.on_device(x.device):
         _native.check(_native.lib().mambo_quantize_mxfp8(
             x.data_ptr(), dtype, m, k, x.stride(0), values.data_ptr(), values.stride(0),
             scales.data_ptr(), scales.stride(0), _native.stream_handle(stream)), "launch_quantize_fp8")

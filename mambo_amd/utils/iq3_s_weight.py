@@ -92,7 +92,7 @@ def prepare_iq3_s_fields(iq3_weight: torch.Tensor, *, fields: bool = True, pack:
     n, blocks = _check_raw(iq3_weight)
     dev = iq3_weight.device
     L = _native.lib()
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         packed = torch.empty(packed_bytes(n, blocks), dtype=torch.uint8, device=dev) if pack or not fields else None
         if fields:
             d = torch.empty((blocks, n), dtype=torch.float16, device=dev)
@@ -189,7 +189,7 @@ def ensure_packed(iq3_weight: IQ3SFields, stream=None) -> torch.Tensor:
     dev = iq3_weight.d.device
     packed = torch.empty(packed_bytes(n, blocks), dtype=torch.uint8, device=dev)
     L = _native.lib()
-    with torch.cuda.device(dev):
+    with _native.on_device(dev):
         _native.check(L.mambo_iq3s_pack(*(t.data_ptr() for t in _weight_kernel_args(iq3_weight)), n, blocks,
                                         packed.data_ptr(), _native.stream_handle(stream)), "pack")
     object.__setattr__(iq3_weight, "packed", packed)

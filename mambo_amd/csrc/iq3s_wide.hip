@@ -21,7 +21,7 @@
 // activation fragment of sub-tile mt+1 requested before sub-tile mt's second MFMA), and the
 // block's 16*MT f32 scalings are spread over the last and the next block's first step. The
 // packed words of the next block are requested as soon as their registers' last code is
-// decoded (a second block in flight measured no faster). 230 VGPRs at MT = 4, so two waves
+// decoded (a second block in flight measured no faster). 233 to 244 VGPRs at MT = 4, so two waves
 // per SIMD; what bounds it there is the power limit (1.7 GHz at 55% MFMA busy at 8192 tokens)
 // and, up to a few hundred tokens, the latency of a step's dependent chain.
 //
@@ -43,6 +43,7 @@
 // 398; 10240 x 8192 at 512 112 -> 90; 8192 x 28672 at 40 / 192 / 512 77 -> 43, 140 -> 102, 230 ->
 // 201; 28672 x 4096 at 2048 441 -> 401; 6204 x 2816 at 128 26 -> 18; 1280 x 8192 at 64 16 -> 12.
 #include "iq3s_wide.h"
+#include "iq3s_wide_copies.h"
 
 #include "iq3s_dense.h"
 
@@ -171,25 +172,16 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
     const uint32_t o16 = second + 16u * rl, o8 = second + 8u * rl, o2 = second + 2u * rl, o1 = second + rl,
                    od = second + 2u * col;
 
-    // Resources that end with row M-1: copies of rows past it are out of range and read
-    // nothing (their outputs are never stored).
-    const auto rows_rsrc = [&](const uint8_t *base, int64_t ld, int row_bytes) {
-        const uint64_t bytes = (uint64_t)(M - 1 - m0) * (uint64_t)ld + (uint64_t)row_bytes;
-        const uint32_t n = (bytes >> 32) ? 0xFFFFFFFFu : (uint32_t)bytes;
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base + m0 * ld), 0,
-                                                 __builtin_amdgcn_readfirstlane((int)n), 0x00020000);
-    };
-    const __amdgpu_buffer_rsrc_t xrows = rows_rsrc(xv, ldxv, B * 256), srows = rows_rsrc(xs, ldxs, B * 8);
+    // Rows past M read row M-1 (their outputs are never stored), by offsets made once
+    // (iq3s_wide_copies.h).
+    const __amdgpu_buffer_rsrc_t xrows = byte_rsrc(xv + m0 * ldxv), srows = byte_rsrc(xs + m0 * ldxs);
+    const int last_row = (int)min<int64_t>(M - 1 - m0, kRows - 1);
     const int srow = wave & (MT - 1); // waves past MT repeat a scale copy (the same bytes): no branch
-    // copy j covers rows 4 * (wave + W * j) .. + 3; with fewer than four waves the swizzle of a lane's
-    // chunk repeats every 4 / W copies
-    constexpr int kSwizzles = W < 4 ? 4 / W : 1;
-    uint32_t voff[kSwizzles];
+    uint32_t voff[kVCopies];
 #pragma unroll
-    for (int j = 0; j < kSwizzles; ++j)
-        voff[j] = (uint32_t)(4 * wave + (lane >> 4)) * (uint32_t)ldxv +
-                  16u * (uint32_t)((lane & 15) ^ ((4 * (wave + W * j) + (lane >> 4)) & 15));
-    const uint32_t soff_stage = (uint32_t)(32 * srow + (lane >> 1)) * (uint32_t)ldxs + 4u * (lane & 1);
+    for (int j = 0; j < kVCopies; ++j)
+        voff[j] = wide_value_offset(wave, lane, W, j, last_row, (uint32_t)ldxv);
+    const uint32_t soff_stage = wide_scale_offset(srow, lane, last_row, (uint32_t)ldxs);
 
     const uint32_t a0 = (uint32_t)(kg * kRows * 256) + 256u * r32 + 16u * (uint32_t)(g ^ col);
     const uint32_t soff = (uint32_t)(kg * kRows * 8) + 8u * r32 + 2u * g;
@@ -211,9 +203,9 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
     auto stage = [&](uint8_t *vals, uint8_t *scl, int b) {
 #pragma unroll
         for (int j = 0; j < kVCopies; ++j) {
-            const uint32_t vo = voff[j % kSwizzles]; // (the host pass drops the kernel with the element as an argument)
+            const uint32_t vo = voff[j]; // (the host pass drops the kernel with the element as an argument)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xrows, (lds_ptr)(vals + kg * kRows * 256 + 1024 * (wave + W * j)),
-                                                     16, vo, 256u * b + (uint32_t)(4 * W * j) * (uint32_t)ldxv, 0, 0);
+                                                     16, vo, 256u * b, 0, 0);
         }
         __builtin_amdgcn_raw_ptr_buffer_load_lds(srows, (lds_ptr)(scl + kg * kRows * 8 + 256 * srow), 4, soff_stage, 8u * b, 0, 0);
     };

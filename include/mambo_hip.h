@@ -52,13 +52,17 @@ enum {
     MAMBO_GEMM_AUTO = 0,    /* library default for the shape */
     MAMBO_GEMM_STREAM = 1,  /* weight-streaming kernel, block-diagonal activations (M <= 4 per MFMA) */
     MAMBO_GEMM_TILED = 2,   /* LDS-tiled kernel for large M */
-    MAMBO_GEMM_DENSE = 3    /* weight-streaming kernel, dense 16-token activations, exact two-term weights */
+    MAMBO_GEMM_DENSE = 3,   /* weight-streaming kernel, dense 16-token activations, exact two-term weights */
+    MAMBO_GEMM_WIDE = 4     /* 32 x 32 MFMA kernel for 33 tokens and more: what mambo_gemm_plan reports of a
+                               call that AUTO gives to it; not a family that a configuration can name */
 };
 
 /* Tunable launch configuration of mambo_iq3s_fp8_matmul (the autotuner's search
  * space; replaces the cuTile tile_m/tile_n/split_k/occupancy hints of
- * iq3_s_fp8.py:49-58,402-465). Zero fields (and kernel == MAMBO_GEMM_AUTO) take the
- * value of mambo_gemm_default_config for the shape. */
+ * iq3_s_fp8.py:49-58,402-465). A configuration with every field zero leaves the choice to the
+ * library, as NULL does (mambo_gemm_plan says what it is). One that names a family or sets a field
+ * takes the value of that family's default (of mambo_gemm_default_config where kernel ==
+ * MAMBO_GEMM_AUTO) in its zero fields. */
 typedef struct mambo_gemm_config {
     int32_t kernel;  /* MAMBO_GEMM_* */
     int32_t waves;   /* waves (64 lanes) per workgroup */
@@ -159,8 +163,9 @@ typedef struct mambo_projection {
     int64_t ldo;           /* >= n */
 } mambo_projection;
 
-/* proj[0..count) share xv/xs and K = blocks*256; cfg as for mambo_iq3s_fp8_matmul, with
- * the default computed for the summed N (mambo_gemm_default_config(m, sum of n, ...)). */
+/* proj[0..count) share xv/xs and K = blocks*256; cfg as for mambo_iq3s_fp8_matmul. What the
+ * library chooses where cfg leaves it to it depends on the summed N and, through the workgroups
+ * that each projection's own rows take, on the N of each (mambo_gemm_plan). */
 int mambo_iq3s_fp8_matmul_grouped(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t ldxs,
                                   int64_t m, const mambo_projection *proj, int count, int64_t blocks,
                                   const mambo_gemm_config *cfg, mambo_stream_t stream);
@@ -244,12 +249,22 @@ int mambo_iq3s_matmul_quantize_grouped_noalloc(const void *x, int x_dtype, int64
                                                const mambo_projection *proj, int count, int64_t blocks,
                                                const mambo_gemm_config *cfg, mambo_stream_t stream);
 
-/* The configuration mambo_iq3s_fp8_matmul uses when cfg == NULL (or all zero), except where
- * another is the faster one for the call's shape: from 5 tokens the tiled kernel's small tiles
- * without a K split (mambo_amd/csrc/iq3s_gemm.hip, small_tiles), from 33 tokens the 32 x 32
- * MFMA kernel (mambo_amd/csrc/iq3s_wide.hip), which splits K only where this configuration
- * does and is not one that a caller can name. */
+/* A named-family configuration for the shape (n: the summed N), which the zero fields of a
+ * configuration take. It is not what cfg == NULL runs wherever another is faster: from 5 tokens the
+ * tiled kernel's small tiles without a K split (mambo_amd/csrc/iq3s_gemm.hip, small_tiles), from 33
+ * tokens the 32 x 32 MFMA kernel (mambo_amd/csrc/iq3s_wide.hip), which splits K only where this
+ * configuration does. A caller that passes this configuration back gets this kernel; to get the
+ * library's choice, pass NULL. */
 int mambo_gemm_default_config(int64_t m, int64_t n, int64_t blocks, mambo_gemm_config *out);
+
+/* What mambo_iq3s_fp8_matmul_grouped (count == 1: mambo_iq3s_fp8_matmul) launches for a call
+ * whose operands are aligned as it asks (x_scales to 8 bytes), on the host alone: of proj only n is read. out:
+ * kernel (MAMBO_GEMM_WIDE among them), waves per workgroup, K slices (split_k; more than one: f32
+ * atomics), tokens (tile_m) and weight rows (tile_n) per workgroup as in mambo_gemm_config; a WIDE
+ * workgroup has waves / (tile_n / 32) K groups. Returns the status that the call would return
+ * for its shape, strides and configuration. */
+int mambo_gemm_plan(int64_t m, const mambo_projection *proj, int count, int64_t blocks, int64_t ldxv,
+                    int64_t ldxs, const mambo_gemm_config *cfg, mambo_gemm_config *out);
 
 /* Validates cfg for the shape (MAMBO_OK or MAMBO_ERR_VALUE with a reason). */
 int mambo_gemm_check_config(int64_t m, int64_t n, int64_t blocks, const mambo_gemm_config *cfg);

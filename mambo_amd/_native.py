@@ -30,6 +30,7 @@ GEMM_AUTO = 0
 GEMM_STREAM = 1
 GEMM_TILED = 2
 GEMM_DENSE = 3
+GEMM_WIDE = 4  # reported by mambo_gemm_plan only
 
 
 class GemmConfig(ctypes.Structure):
@@ -115,6 +116,8 @@ SIGNATURES = {
                                            _vp, _vp]),
     "mambo_chain_status": (_i32, [_vp]),
     "mambo_gemm_default_config": (_i32, [_i64, _i64, _i64, ctypes.POINTER(GemmConfig)]),
+    "mambo_gemm_plan": (_i32, [_i64, ctypes.POINTER(Projection), _i32, _i64, _i64, _i64, ctypes.POINTER(GemmConfig),
+                               ctypes.POINTER(GemmConfig)]),
     "mambo_gemm_check_config": (_i32, [_i64, _i64, _i64, ctypes.POINTER(GemmConfig)]),
     "mambo_gemm_config_enumerate": (_i64, [_i64, _i64, _i64, ctypes.POINTER(GemmConfig), _i64]),
     "mambo_synth_iq3s": (_i32, [_u64, _i64, _i64, _i64, _vp, _vp]),

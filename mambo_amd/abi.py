@@ -169,6 +169,11 @@ CONSTRAINTS: dict[str, list[dict]] = {
     ],
     "mambo_chain_status": [_arr("sync", "uint32", ["MAMBO_CHAIN_SYNC_WORDS"], align=4, access="readwrite")],
     "mambo_gemm_default_config": [_arr("out", "mambo_gemm_config", ["1"], align=4, memory="host", access="write")],
+    "mambo_gemm_plan": [
+        _arr("proj", "mambo_projection", ["count"], align=8, memory="host"),
+        _arr("cfg", "mambo_gemm_config", ["1"], align=4, memory="host", nullable=True),
+        _arr("out", "mambo_gemm_config", ["1"], align=4, memory="host", access="write"),
+    ],
     "mambo_gemm_check_config": [_arr("cfg", "mambo_gemm_config", ["1"], align=4, memory="host")],
     "mambo_gemm_config_enumerate": [
         _arr("out", "mambo_gemm_config", ["capacity"], align=4, memory="host", nullable=True, access="write")],

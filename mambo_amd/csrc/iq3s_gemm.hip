@@ -2022,14 +2022,16 @@ bool small_tiles(int64_t m, const mambo_projection *proj, int count, int64_t blo
     return found;
 }
 
-// quant: -1 when xv/xs are MXFP8 activations; else xv holds unquantized rows of dtype
-// quant (ldxv in elements, xs unused) for the stream kernel to quantize itself, and the
-// call returns kNotFused, launching nothing, when the configuration cannot do that.
-int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t ldxs, int64_t m,
-                    const mambo_projection *proj, int count, int64_t blocks, const mambo_gemm_config *cfg,
-                    hipStream_t s, int quant = -1)
+// What a call launches: the 32 x 32 MFMA kernel by `plan`, else configuration c.
+struct Choice {
+    bool wide;
+    WidePlan plan;
+    mambo_gemm_config c;
+};
+
+// The shape and stride checks of a call (quant as for run_projections).
+int check_call(int64_t m, int count, int64_t blocks, int64_t ldxv, int64_t ldxs, int quant)
 {
-    MAMBO_REQUIRE(xv && (xs || quant >= 0) && proj, MAMBO_ERR_VALUE, "null pointer");
     MAMBO_REQUIRE(count >= 1 && count <= kMaxGroup, MAMBO_ERR_VALUE, "count must be in [1, %d] (got %d)", kMaxGroup,
                   count);
     MAMBO_REQUIRE(m >= 1 && blocks >= 1, MAMBO_ERR_VALUE, "shape must be positive (M=%lld B=%lld)", (long long)m,
@@ -2040,12 +2042,75 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
                   "activation row strides must cover the row");
     MAMBO_REQUIRE(ldxv < ((int64_t)1 << 27) && (quant >= 0 || ldxs < ((int64_t)1 << 27)), MAMBO_ERR_VALUE,
                   "activation row stride too large");
+    return MAMBO_OK;
+}
+
+// Which kernel takes a call of those shapes (of each projection only n is read), and how.
+int choose(int64_t m, const mambo_projection *proj, int count, int64_t blocks, int64_t ldxv, const uint8_t *xs,
+           int64_t ldxs, const mambo_gemm_config *cfg, int quant, Choice *out)
+{
+    int64_t n_total = 0;
+    for (int g = 0; g < count; ++g)
+        n_total += proj[g].n;
+    out->wide = false;
+    mambo_gemm_config &c = out->c;
+    // Library default of the requested kernel family (or of the family chosen by M),
+    // overlaid with the non-zero fields of cfg.
+    MAMBO_REQUIRE(cfg == nullptr || (cfg->kernel >= MAMBO_GEMM_AUTO && cfg->kernel <= MAMBO_GEMM_DENSE),
+                  MAMBO_ERR_VALUE, "unsupported kernel family %d", cfg ? cfg->kernel : 0);
+    c = family_default(cfg ? cfg->kernel : MAMBO_GEMM_AUTO, m, n_total, blocks);
+    if (cfg != nullptr) {
+        if (cfg->waves)
+            c.waves = cfg->waves;
+        if (cfg->split_k)
+            c.split_k = cfg->split_k;
+        if (cfg->tile_m)
+            c.tile_m = cfg->tile_m;
+        if (cfg->tile_n)
+            c.tile_n = cfg->tile_n;
+        const int rc = mambo_gemm_check_config(m, n_total, blocks, &c);
+        if (rc)
+            return rc;
+    }
+    // A call that leaves the configuration to the library takes the 32 x 32 MFMA kernel or small
+    // tiles where they are the faster ones.
+    if (quant < 0 && (cfg == nullptr || all_default(*cfg))) {
+        bool have_wide = mambo_wide_plan(m, proj, count, blocks, ldxv, xs, ldxs, c, &out->plan);
+        double us = have_wide ? out->plan.us : 0.0;
+        // few rows and a long K: the dense kernel's K split (199 x 19712 at 47 tokens 10.5 and 12.7 us)
+        if (!have_wide || (c.kernel == MAMBO_GEMM_DENSE && c.split_k > 1)) {
+            const double base = config_time(c, m, n_total, blocks);
+            have_wide = have_wide && us <= 0.9 * base;
+            us = have_wide ? us : base;
+        }
+        mambo_gemm_config small;
+        if (small_tiles(m, proj, count, blocks, xs, ldxs, c, us, &small) &&
+            mambo_gemm_check_config(m, n_total, blocks, &small) == MAMBO_OK)
+            c = small;
+        else
+            out->wide = have_wide;
+    }
+    return MAMBO_OK;
+}
+
+// quant: -1 when xv/xs are MXFP8 activations; else xv holds unquantized rows of dtype
+// quant (ldxv in elements, xs unused) for the stream kernel to quantize itself, and the
+// call returns kNotFused, launching nothing, when the configuration cannot do that.
+int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t ldxs, int64_t m,
+                    const mambo_projection *proj, int count, int64_t blocks, const mambo_gemm_config *cfg,
+                    hipStream_t s, int quant = -1)
+{
+    MAMBO_REQUIRE(xv && (xs || quant >= 0) && proj, MAMBO_ERR_VALUE, "null pointer");
+    int rc = check_call(m, count, blocks, ldxv, ldxs, quant);
+    if (rc)
+        return rc;
+    const int64_t k = blocks * 256;
     if (quant < 0)
         MAMBO_REQUIRE((uintptr_t)xv % 16 == 0 && ldxv % 16 == 0, MAMBO_ERR_VALUE,
                       "x_values base and row stride must be 16-byte aligned");
     GroupArgs ga = {};
     ga.count = count;
-    int64_t tiles = 0, n_total = 0;
+    int64_t tiles = 0;
     for (int g = 0; g < count; ++g) {
         const mambo_projection &p = proj[g];
         MAMBO_REQUIRE(p.packed && p.out, MAMBO_ERR_VALUE, "projection %d: null pointer", g);
@@ -2058,51 +2123,19 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
         ga.ldo[g] = p.ldo;
         ga.tile_begin[g] = tiles;
         tiles += cdiv(p.n, kTileRows);
-        n_total += p.n;
     }
-    // Library default of the requested kernel family (or of the family chosen by M),
-    // overlaid with the non-zero fields of cfg.
-    MAMBO_REQUIRE(cfg == nullptr || (cfg->kernel >= MAMBO_GEMM_AUTO && cfg->kernel <= MAMBO_GEMM_DENSE),
-                  MAMBO_ERR_VALUE, "unsupported kernel family %d", cfg ? cfg->kernel : 0);
-    mambo_gemm_config c = family_default(cfg ? cfg->kernel : MAMBO_GEMM_AUTO, m, n_total, blocks);
-    int rc = MAMBO_OK;
-    if (cfg != nullptr) {
-        if (cfg->waves)
-            c.waves = cfg->waves;
-        if (cfg->split_k)
-            c.split_k = cfg->split_k;
-        if (cfg->tile_m)
-            c.tile_m = cfg->tile_m;
-        if (cfg->tile_n)
-            c.tile_n = cfg->tile_n;
-        rc = mambo_gemm_check_config(m, n_total, blocks, &c);
-        if (rc)
-            return rc;
-    }
-    // A call that leaves the configuration to the library takes the 32 x 32 MFMA kernel or small
-    // tiles where they are the faster ones.
-    if (quant < 0 && (cfg == nullptr || all_default(*cfg))) {
-        WidePlan wide;
-        bool have_wide = mambo_wide_plan(m, proj, count, blocks, ldxv, xs, ldxs, c, &wide);
-        double us = have_wide ? wide.us : 0.0;
-        // few rows and a long K: the dense kernel's K split (199 x 19712 at 47 tokens 10.5 and 12.7 us)
-        if (!have_wide || (c.kernel == MAMBO_GEMM_DENSE && c.split_k > 1)) {
-            const double base = config_time(c, m, n_total, blocks);
-            have_wide = have_wide && us <= 0.9 * base;
-            us = have_wide ? us : base;
+    Choice choice;
+    rc = choose(m, proj, count, blocks, ldxv, xs, ldxs, cfg, quant, &choice);
+    if (rc)
+        return rc;
+    const mambo_gemm_config &c = choice.c;
+    if (choice.wide) {
+        if (choice.plan.splits > 1) {
+            rc = zero_outputs(ga, m, s);
+            if (rc)
+                return rc;
         }
-        mambo_gemm_config small;
-        if (small_tiles(m, proj, count, blocks, xs, ldxs, c, us, &small) &&
-            mambo_gemm_check_config(m, n_total, blocks, &small) == MAMBO_OK) {
-            c = small;
-        } else if (have_wide) {
-            if (wide.splits > 1) {
-                rc = zero_outputs(ga, m, s);
-                if (rc)
-                    return rc;
-            }
-            return mambo_wide_launch(wide, xv, ldxv, xs, ldxs, m, proj, count, blocks, s);
-        }
+        return mambo_wide_launch(choice.plan, xv, ldxv, xs, ldxs, m, proj, count, blocks, s);
     }
     if (quant >= 0) { // in-kernel quantization: stream kernel, one sub-tile, rows staged in LDS
         const int64_t esz = quant == MAMBO_DTYPE_BF16 ? 2 : 4;
@@ -2166,6 +2199,34 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
 }
 
 } // namespace
+
+extern "C" int mambo_gemm_plan(int64_t m, const mambo_projection *proj, int count, int64_t blocks, int64_t ldxv,
+                               int64_t ldxs, const mambo_gemm_config *cfg, mambo_gemm_config *out)
+{
+    MAMBO_REQUIRE(proj && out, MAMBO_ERR_VALUE, "null pointer");
+    int rc = check_call(m, count, blocks, ldxv, ldxs, -1);
+    if (rc)
+        return rc;
+    for (int g = 0; g < count; ++g)
+        MAMBO_REQUIRE(proj[g].n >= 1, MAMBO_ERR_VALUE, "projection %d: n must be positive (N=%lld)", g,
+                      (long long)proj[g].n);
+    Choice choice;
+    rc = choose(m, proj, count, blocks, ldxv, nullptr, ldxs, cfg, -1, &choice);
+    if (rc)
+        return rc;
+    *out = choice.c;
+    out->split_k = (int32_t)cdiv(blocks, cdiv(blocks, choice.c.split_k));
+    if (choice.wide) {
+        const WidePlan &p = choice.plan;
+        *out = {};
+        out->kernel = MAMBO_GEMM_WIDE;
+        out->waves = p.waves * p.kg;
+        out->split_k = p.splits;
+        out->tile_m = 32 * p.mt;
+        out->tile_n = 32 * p.waves;
+    }
+    return MAMBO_OK;
+}
 
 extern "C" int mambo_iq3s_fp8_matmul(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t ldxs, int64_t m,
                                      const uint8_t *packed, int64_t n, int64_t blocks, float *out, int64_t ldo,

@@ -346,6 +346,7 @@ const std::vector<EntryDecl> &compiled_entries()
         MAMBO_ENTRY(mambo_iq3s_fp8_matmul_chain, "m", "launches", "count", "cfg", "sync", "stream"),
         MAMBO_ENTRY(mambo_chain_status, "sync"),
         MAMBO_ENTRY(mambo_gemm_default_config, "m", "n", "blocks", "out"),
+        MAMBO_ENTRY(mambo_gemm_plan, "m", "proj", "count", "blocks", "ldxv", "ldxs", "cfg", "out"),
         MAMBO_ENTRY(mambo_gemm_check_config, "m", "n", "blocks", "cfg"),
         MAMBO_ENTRY(mambo_gemm_config_enumerate, "m", "n", "blocks", "out", "capacity"),
         MAMBO_ENTRY(mambo_synth_iq3s, "seed", "blocks", "row0", "nrows", "raw", "stream"),

@@ -1,0 +1,48 @@
+"""mambo_gemm_plan (no GPU): what a projection call launches, and what it refuses."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+from plan import plan, raw_plan
+
+
+def test_plan_reports_the_kernel_of_a_call():
+    from mambo_amd import _native
+    # a named configuration comes back as it runs, its zero fields filled, its K slices counted
+    named = {"kernel": _native.GEMM_TILED, "waves": 8, "tile_m": 64, "tile_n": 128, "split_k": 5}
+    assert plan(512, [4096], 16, config=named) == {**named, "split_k": 4}
+    assert plan(1, [4096], 16)["kernel"] == _native.GEMM_STREAM
+    # the library's choice from 33 tokens: 128 x 256 tiles, and none of a family's configurations
+    wide = plan(2048, [28672], 16)
+    assert wide == {"kernel": _native.GEMM_WIDE, "waves": 8, "split_k": 1, "tile_m": 128, "tile_n": 256}
+    default = _native.GemmConfig()
+    assert _native.lib().mambo_gemm_default_config(2048, 28672, 16, ctypes.byref(default)) == 0
+    assert default.kernel != _native.GEMM_WIDE
+    assert plan(2048, [28672], 16, config=default.as_dict()) == default.as_dict()
+    # few workgroups: small tiles of the tiled kernel, no K split
+    small = plan(128, [1024], 16)
+    assert (small["kernel"], small["split_k"]) == (_native.GEMM_TILED, 1) and small["tile_m"] <= 32
+    # by the N of each projection, not by their sum alone
+    assert plan(128, [16384], 16)["tile_m"] == 64 and plan(128, [16192, 64, 64, 64], 16)["tile_m"] == 128
+
+
+def test_plan_refuses_what_the_call_refuses():
+    from mambo_amd import _native
+    lib, err = _native.lib(), _native.MAMBO_ERR_VALUE
+    out = _native.GemmConfig()
+    one = (_native.Projection * 1)(_native.Projection(0, 64, 0, 64))
+    assert lib.mambo_gemm_plan(1, None, 1, 4, 1024, 32, None, ctypes.byref(out)) == err
+    assert lib.mambo_gemm_plan(1, one, 1, 4, 1024, 32, None, None) == err
+    for m, ns, blocks, kwargs, text in (
+            (0, [64], 4, {}, "positive"), (1, [0], 4, {}, "n must be positive"), (1, [64] * 5, 4, {}, "count"),
+            (64, [64], 4, {"ldxv": 1008}, "cover the row"), (64, [64], 4, {"ldxs": 24}, "cover the row"),
+            (64, [64], 4, {"ldxv": 1 << 27}, "stride too large"),
+            (64, [64], 4, {"config": {"kernel": _native.GEMM_WIDE}}, "unsupported kernel family"),
+            (64, [64], 4, {"config": {"kernel": _native.GEMM_TILED, "waves": 3}}, "waves")):
+        rc, _ = raw_plan(m, ns, blocks, **kwargs)
+        assert rc == err and text in lib.mambo_last_error().decode(), (m, ns, kwargs, lib.mambo_last_error())
+    with pytest.raises(ValueError, match="positive"):
+        plan(0, [64], 4)

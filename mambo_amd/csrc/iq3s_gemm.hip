@@ -2045,6 +2045,13 @@ int check_call(int64_t m, int count, int64_t blocks, int64_t ldxv, int64_t ldxs,
     return MAMBO_OK;
 }
 
+// Whether the staging copies of a tiled configuration reach a token tile's rows with 32-bit offsets.
+bool tile_offsets_fit(const mambo_gemm_config &c, int64_t ldxv, int64_t ldxs)
+{
+    return c.kernel != MAMBO_GEMM_TILED ||
+           ((int64_t)c.tile_m * ldxv < ((int64_t)1 << 32) && (int64_t)c.tile_m * ldxs < ((int64_t)1 << 32));
+}
+
 // Which kernel takes a call of those shapes (of each projection only n is read), and how.
 int choose(int64_t m, const mambo_projection *proj, int count, int64_t blocks, int64_t ldxv, const uint8_t *xs,
            int64_t ldxs, const mambo_gemm_config *cfg, int quant, Choice *out)
@@ -2073,8 +2080,8 @@ int choose(int64_t m, const mambo_projection *proj, int count, int64_t blocks, i
             return rc;
     }
     // A call that leaves the configuration to the library takes the 32 x 32 MFMA kernel or small
-    // tiles where they are the faster ones.
-    if (quant < 0 && (cfg == nullptr || all_default(*cfg))) {
+    // tiles where they are the faster ones (not one with row strides that c's tile refuses).
+    if (quant < 0 && (cfg == nullptr || all_default(*cfg)) && tile_offsets_fit(c, ldxv, ldxs)) {
         bool have_wide = mambo_wide_plan(m, proj, count, blocks, ldxv, xs, ldxs, c, &out->plan);
         double us = have_wide ? out->plan.us : 0.0;
         // few rows and a long K: the dense kernel's K split (199 x 19712 at 47 tokens 10.5 and 12.7 us)
@@ -2090,6 +2097,9 @@ int choose(int64_t m, const mambo_projection *proj, int count, int64_t blocks, i
         else
             out->wide = have_wide;
     }
+    if (quant < 0 && !out->wide)
+        MAMBO_REQUIRE(tile_offsets_fit(c, ldxv, ldxs), MAMBO_ERR_VALUE,
+                      "tiled: activation row stride too large for tile_m=%d", c.tile_m);
     return MAMBO_OK;
 }
 
@@ -2161,9 +2171,6 @@ int run_projections(const uint8_t *xv, int64_t ldxv, const uint8_t *xs, int64_t 
         const int mt = c.tile_m / 16, nt = c.tile_n / (16 * tw);
         MAMBO_REQUIRE((uintptr_t)xs % 8 == 0 && ldxs % 8 == 0, MAMBO_ERR_VALUE,
                       "tiled: x_scales base and row stride must be 8-byte aligned");
-        // the staging copies address a token tile with 32-bit offsets
-        MAMBO_REQUIRE((int64_t)c.tile_m * ldxv < ((int64_t)1 << 32) && (int64_t)c.tile_m * ldxs < ((int64_t)1 << 32),
-                      MAMBO_ERR_VALUE, "tiled: activation row stride too large for tile_m=%d", c.tile_m);
         // workgroups per projection; tile_begin counts workgroups for this kernel
         GroupArgs gt = ga;
         int64_t wgs = 0;

@@ -488,9 +488,10 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
                      const uint8_t *xs, int64_t ldxs, const mambo_gemm_config &other, WidePlan *plan)
 {
     // what the kernel's addressing assumes: scale rows copied as dwords (8-byte aligned, as the
-    // tiled kernel asks), a token tile within 32-bit offsets, grid limits
+    // tiled kernel asks), a token tile's values and scales within 32-bit offsets, grid limits
     if (m < 33 || blocks < 4 || (uintptr_t)xs % 8 != 0 || ldxs % 8 != 0 ||
-        256 * ldxv + blocks * 256 >= ((int64_t)1 << 32) || cdiv(m, 64) > 65535)
+        256 * ldxv + blocks * 256 >= ((int64_t)1 << 32) || 256 * ldxs + blocks * 8 >= ((int64_t)1 << 32) ||
+        cdiv(m, 64) > 65535)
         return false;
     int64_t n = 0;
     for (int g = 0; g < count; ++g)

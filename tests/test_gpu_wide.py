@@ -161,3 +161,20 @@ def test_wide_same_bits_without_a_split_and_under_capture(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), first)
+
+
+def test_scale_rows_beyond_32_bit_offsets(gpu):
+    """Rows of scales so far apart that 63 of them pass 4 GiB: not for tiles with 32-bit offsets."""
+    from mambo_amd.kernels.iq3_s_fp8 import launch_iq3_s_fp8_matmul
+    from mambo_amd.utils.iq3_s_weight import prepare_iq3_s_fields
+    m, n, blocks, ld = 63, 12304, 4, (1 << 32) // 62 // 8 * 8 + 8
+    k = 256 * blocks
+    raw = make_synthetic_iq3_s(n, k, seed=5)
+    xv, xs = oracle.quantize_mxfp8(np.random.default_rng(5).standard_normal((m, k)).astype(np.float32))
+    w = prepare_iq3_s_fields(torch.from_numpy(raw).to(gpu), fields=False)
+    far = torch.empty(m * ld, dtype=torch.uint8, device=gpu).as_strided((m, k // 32), (ld, 1))
+    far.copy_(torch.from_numpy(xs).to(gpu))
+    step(f"scale rows {ld} bytes apart")
+    out = launch_iq3_s_fp8_matmul(torch.from_numpy(xv).to(gpu), far, w, config={"kernel": 0}).cpu().numpy()
+    rows = np.random.default_rng(1).choice(n, 64, replace=False)
+    assert rel_l2(out[:, rows], oracle.iq3s_fp8_matmul(xv, xs, raw[rows], threads=oracle.default_threads())) < 1e-4

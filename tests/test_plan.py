@@ -46,3 +46,23 @@ def test_plan_refuses_what_the_call_refuses():
         assert rc == err and text in lib.mambo_last_error().decode(), (m, ns, kwargs, lib.mambo_last_error())
     with pytest.raises(ValueError, match="positive"):
         plan(0, [64], 4)
+
+
+def test_plan_strides_within_32_bit_offsets():
+    """The copies of a token tile address its rows with 32-bit offsets, values and scales alike. A call
+    whose row strides do not fit a kernel's tile goes to one whose tile they fit, and is
+    refused where the named default's tile is too tall for them."""
+    from mambo_amd import _native
+    top = (1 << 27) - 16  # strides end below 2^27
+    for name, unit in (("ldxv", 16), ("ldxs", 8)):
+        for m, ns, blocks in ((2048, [28672], 16), (128, [8192], 112), (48, [28672], 16), (300, [4096], 112)):
+            assert plan(m, ns, blocks)["kernel"] == _native.GEMM_WIDE
+            default = _native.GemmConfig()
+            _native.check(_native.lib().mambo_gemm_default_config(m, sum(ns), blocks, ctypes.byref(default)))
+            for ld in sorted({unit * (x // unit) + d * unit for s in range(20, 27) for d in (-1, 0, 1)
+                              for x in (1 << s, (1 << s) * 33 // 32)} | {top}):
+                rc, p = raw_plan(m, ns, blocks, **{name: ld})
+                fits = default.kernel != _native.GEMM_TILED or default.tile_m * ld < 1 << 32
+                assert (rc == 0) == fits, (m, name, ld)
+                if rc == 0 and p.kernel in (_native.GEMM_WIDE, _native.GEMM_TILED):
+                    assert (p.tile_m - 1) * ld + 256 * blocks < 1 << 32, (m, name, ld, p.as_dict())

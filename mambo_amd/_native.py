@@ -202,10 +202,15 @@ _here = nullcontext()
 
 def on_device(device):
     """Context with `device` (a tensor's) current; nothing to do where it is already, as in most
-    calls: entering and leaving torch.cuda.device costs an eager call about 2 us."""
+    calls: entering and leaving torch.cuda.device costs an eager call about 2 us. An exchange with
+    itself and not torch.cuda.current_device tells: that one may report a device that torch has
+    still to switch the runtime to, and the exchange does so."""
     import torch
-    if device.type == "cuda" and device.index == torch.cuda.current_device():
-        return _here
+    if device.type == "cuda":
+        before = torch.cuda._exchange_device(device.index)
+        if before == device.index:
+            return _here
+        torch.cuda._maybe_exchange_device(before)
     return torch.cuda.device(device)
 
 

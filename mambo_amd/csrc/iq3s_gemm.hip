@@ -2000,7 +2000,7 @@ bool small_tiles(int64_t m, const mambo_projection *proj, int count, int64_t blo
         n += proj[g].n;
     const double mn = (double)m * (double)n;
     double best = 0.97 * other_us;
-    bool found = false;
+    int64_t best_wgs = 0;
     for (const Tile &t : kTiles) {
         int64_t wgs = 0;
         for (int g = 0; g < count; ++g)
@@ -2016,10 +2016,18 @@ bool small_tiles(int64_t m, const mambo_projection *proj, int count, int64_t blo
             out->split_k = 1;
             out->tile_m = t.tokens;
             out->tile_n = t.rows;
-            found = true;
+            best_wgs = wgs;
         }
     }
-    return found;
+    // Up to 10 tokens a dense kernel whose four waves divide K streams the weights as fast, and
+    // faster than 64-row tiles that leave a CU one workgroup (us, dense and tiles: 15692 x 16384 at 5 /
+    // 7 / 9 tokens 31.3, 32.5, 34.5 and 38.0, 37.7, 37.4; 16005 x 18432 at 5 35.6 and 43.1; 15646 x
+    // 6144 at 5 14.2 and 15.2) or, on a long K, two (28569 x 16384 at 5 57.6 and 61.7). From 11 the
+    // tiles are ahead there too (16018 x 13312 at 16 35.2 and 30.9).
+    if (best_wgs > 0 && m <= 10 && out->tile_n == 64 && other.kernel == MAMBO_GEMM_DENSE && other.split_k == 1 &&
+        other.waves >= 4 && best_wgs <= (blocks >= 48 ? 2 * kCUs : kCUs))
+        return false;
+    return best_wgs > 0;
 }
 
 // What a call launches: the 32 x 32 MFMA kernel by `plan`, else configuration c.

@@ -500,7 +500,8 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
     // either side): wherever the other plan splits K (64 tokens and more; 1-35%), so that sums
     // that were in a fixed order stay so; against an unsplit tiled plan from 9 K blocks on
     // (4-35%; on 4 and 8 blocks launches of 7-17 us, the 64-token tiles are 1-12% ahead) or
-    // where 128 x 128 tiles give every CU one; against the dense kernel (which decodes a weight
+    // where 128 x 128 tiles give every CU one, but on 4 blocks not where the other's 64 x 128 tiles are
+    // a single round of two per CU (8192 x 1024 at 400 tokens 13.1 and 14.7); against the dense kernel (which decodes a weight
     // once per 32 tokens) where 64 x 128 tiles take 80 CUs (us at 40 tokens: 28672
     // x 4096 46 against 25, 14336 x 8192 43 and 36, 10240 x 4096 21.3 and 20.1; 8192 x 4096,
     // 64 workgroups, 16.3 and 19.9), or where its waves do not divide few K blocks and it takes 64
@@ -511,12 +512,17 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
     if (!split) {
         const int64_t wgs64 = row_wgs * cdiv(m, 64);
         if (other.kernel == MAMBO_GEMM_DENSE ? !(wgs64 >= 80 || (blocks % 4 != 0 && blocks <= 11 && other.tile_n >= 64))
-                                             : !(blocks >= 9 || fills))
+                                             : !(blocks >= 9 || fills) ||
+                                                   (blocks == 4 && other.tile_m == 64 && wgs64 <= 2 * kCUs))
             return false;
     }
     const double mb = 4e-6 * (double)m * (double)n;
     double best = 0.0;
     for (const WideShape &w : kWideShapes) {
+        // eight waves from 9 blocks on: four of them on 128 x 128 tiles are 4-17% faster before
+        // (7383 x 1280 at 959 tokens 30.6 and 25.6, 22818 x 2048 at 921 112 and 102)
+        if (w.waves == 8 && blocks < 9)
+            continue;
         // 64-token tiles decode each weight twice as often: only while 128-token ones leave CUs
         // idle, or where they pad away most of the last tile
         if (w.mt == 2 && fills && (m % 128 == 0 || m % 128 > 64))

@@ -66,3 +66,20 @@ def test_plan_strides_within_32_bit_offsets():
                 assert (rc == 0) == fits, (m, name, ld)
                 if rc == 0 and p.kernel in (_native.GEMM_WIDE, _native.GEMM_TILED):
                     assert (p.tile_m - 1) * ld + 256 * blocks < 1 << 32, (m, name, ld, p.as_dict())
+
+
+def test_plan_where_the_named_default_is_the_faster():
+    """Launches that the small tiles and the 32 x 32 kernel leave to the named default, and the other
+    side of each line."""
+    from mambo_amd import _native
+    dense, tiled, wide = _native.GEMM_DENSE, _native.GEMM_TILED, _native.GEMM_WIDE
+    # up to 10 tokens, 64-row tiles of one workgroup per CU, or of two on a long K
+    assert [plan(m, [15692], 64)["kernel"] for m in (5, 10, 11)] == [dense, dense, tiled]
+    assert [plan(m, [28569], 64)["kernel"] for m in (5, 10, 11)] == [dense, dense, tiled]
+    assert plan(5, [28672], 32)["kernel"] == tiled  # two on a shorter K
+    assert plan(8, [14336], 32)["tile_n"] == 32 and plan(8, [14336], 32)["kernel"] == tiled
+    # four K blocks where 64-token tiles are one round of two workgroups per CU
+    assert plan(400, [8192], 4) == {"kernel": tiled, "waves": 8, "split_k": 1, "tile_m": 64, "tile_n": 128}
+    assert plan(400, [10240], 4)["kernel"] == wide and plan(400, [8192], 5)["kernel"] == wide
+    # eight waves of 32 rows from nine K blocks
+    assert plan(960, [7383], 8)["tile_n"] == 128 and plan(960, [28672], 9)["tile_n"] == 256

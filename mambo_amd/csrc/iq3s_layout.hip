@@ -284,18 +284,17 @@ __global__ __launch_bounds__(256) void pack_fields_kernel(SoaSrc src, int64_t n,
         pack_lane(FieldBlock{src, b * n + row, row < n}, lane, packed + (t * blocks + b) * (int64_t)kTileBytes);
 }
 
-// 32 rows x 4 blocks per workgroup, 16 values (half a weight group) per thread, row and block.
+// Rows x Blocks per workgroup, 16 values (half a weight group) per thread, 16 rows and block.
 // Memory-bound (110 bytes in, 288 out per block), so what counts is whole lines: a store of the
 // wave covers 1 KiB of values without holes (a thread with the 32 values of a group stored every
-// second 16 bytes, twice), the scales of a row leave in one piece of 128 bytes, and a
-// field of a block is read in runs of 32 rows (2 KiB of qs). With whole lines the nontemporal
+// second 16 bytes, twice), the scales of a row leave in one piece of up to 128 bytes, and a
+// field of a block is read in runs of Rows rows (2 KiB of qs for 32). With whole lines the nontemporal
 // hint pays: nothing written is read here again. Workgroups next to each other take blocks of the same rows.
-// Thread per group -> halves -> halves, nontemporal (us): 4096 x 14336 30.7 -> 22.2 -> 15.2 (7.4 TB/s; a
+// Thread per group -> halves -> halves, nontemporal (us), 32 x 4: 4096 x 14336 30.7 -> 22.2 -> 15.2 (6.0 TB/s; a
 // copy moves 4.8), 28672 x 4096 57 -> 40 -> 28, 8192 x 28672 107 -> 79 -> 54, 4096 x 4096 7.2 -> 6.4 ->
-// 5.8, 1024 x 4096 4.2 -> 4.2 -> 4.1. Rows before blocks in the launch 1-6% slower at 4096 columns, 16 x 8 the same,
+// 5.8. Rows before blocks in the launch 1-6% slower at 4096 columns, 16 x 8 the same,
 // 64 x 4 up to 25% slower.
-constexpr int kDequantRows = 32, kDequantBlocks = 4;
-
+template <int Rows, int Blocks>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict__ d, const uint32_t *__restrict__ qs,
                                                       const uint16_t *__restrict__ qh,
                                                       const int32_t *__restrict__ signs,
@@ -304,34 +303,35 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict
                                                       float *__restrict__ out_scales)
 {
     __shared__ uint32_t lut[512];
-    constexpr int kPasses = kDequantRows / 16;
-    static_assert(kDequantRows * kDequantBlocks * 2 == 256, "a thread writes four scales");
+    constexpr int kPasses = Rows / 16, kPieces = 2 * Blocks; // kPieces: four scales each, of a row
+    static_assert(Rows % 16 == 0 && Rows * kPieces <= 256, "a thread writes four scales at most");
     const int tid = threadIdx.x, u = tid & 15; // u: half of a group of the thread's row
     for (int i = tid; i < 512; i += 256)
         lut[i] = c_grid.fp8[i];
-    const int64_t row0 = (int64_t)(blockIdx.x / groups) * kDequantRows;
-    const int64_t b0 = (int64_t)(blockIdx.x % groups) * kDequantBlocks;
+    const int64_t row0 = (int64_t)(blockIdx.x / groups) * Rows;
+    const int64_t b0 = (int64_t)(blockIdx.x % groups) * Blocks;
     // all loads first; past the weight the last block and row again
     const auto element = [&](int row, int j) { return min(b0 + j, blocks - 1) * n + min(row0 + row, n - 1); };
-    uint32_t q[kPasses][kDequantBlocks], hb[kPasses][kDequantBlocks], sw[kPasses][kDequantBlocks];
+    uint32_t q[kPasses][Blocks], hb[kPasses][Blocks], sw[kPasses][Blocks];
 #pragma unroll
     for (int p = 0; p < kPasses; ++p)
 #pragma unroll
-        for (int j = 0; j < kDequantBlocks; ++j) {
+        for (int j = 0; j < Blocks; ++j) {
             const int64_t e = element(16 * p + (tid >> 4), j);
             q[p][j] = qs[e * 16 + u];
             hb[p][j] = (uint32_t)reinterpret_cast<const uint8_t *>(qh)[e * 8 + (u >> 1)] >> (4 * (u & 1));
             sw[p][j] = reinterpret_cast<const uint16_t *>(signs)[e * 16 + u];
         }
-    // scales: row tid >> 3, half tid & 1 of its block (tid >> 1) & 3
-    const int64_t es = element(tid >> 3, (tid >> 1) & 3);
+    // scales: half tid & 1 of block tid / 2 of row tid / kPieces
+    const int srow = tid / kPieces, sblock = tid % kPieces >> 1;
+    const int64_t es = element(srow, sblock);
     const uint32_t sc = scales[es] >> (16 * (tid & 1));
     const float df = half_bits_to_float(d[es]);
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < kPasses; ++p)
 #pragma unroll
-        for (int j = 0; j < kDequantBlocks; ++j) {
+        for (int j = 0; j < Blocks; ++j) {
             u32x4 out;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -343,14 +343,26 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint16_t *__restrict
             if (row < n && b < blocks)
                 __builtin_nontemporal_store(out, reinterpret_cast<u32x4 *>(values + (row * blocks + b) * 256) + u);
         }
-    const int64_t row = row0 + (tid >> 3), b = b0 + ((tid >> 1) & 3);
-    if (row < n && b < blocks) {
+    const int64_t row = row0 + srow, b = b0 + sblock;
+    if (srow < Rows && row < n && b < blocks) {
         f32x4 out;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             out[i] = df * (float)(1u + 2u * ((sc >> (4 * i)) & 15u));
         *reinterpret_cast<f32x4 *>(out_scales + (row * blocks + b) * 8 + 4 * (tid & 1)) = out;
     }
+}
+
+template <int Rows, int Blocks>
+int launch_dequant(const uint16_t *d, const uint32_t *qs, const uint16_t *qh, const int32_t *signs,
+                   const uint32_t *scales, int64_t n, int64_t blocks, uint8_t *values, float *out_scales,
+                   hipStream_t stream)
+{
+    const int64_t rows = (n + Rows - 1) / Rows, groups = (blocks + Blocks - 1) / Blocks;
+    MAMBO_REQUIRE(rows <= 0x7FFFFFFF / groups, MAMBO_ERR_VALUE, "weight too large");
+    MAMBO_LAUNCH((dequant_kernel<Rows, Blocks>), dim3((unsigned)(rows * groups)), dim3(256), 0, stream, d, qs, qh,
+                 signs, scales, n, blocks, (uint32_t)groups, values, out_scales);
+    return mambo_check_launch("iq3s_dequant");
 }
 
 } // namespace
@@ -414,9 +426,9 @@ extern "C" int mambo_iq3s_dequant(const uint16_t *d, const uint32_t *qs, const u
     MAMBO_REQUIRE(d && qs && qh && signs && scales && values && out_scales, MAMBO_ERR_VALUE, "null pointer");
     MAMBO_REQUIRE(n >= 1 && blocks >= 1, MAMBO_ERR_VALUE, "IQ3_S weight must have positive N and K");
     MAMBO_REQUIRE((uintptr_t)values % 16 == 0, MAMBO_ERR_VALUE, "values must be 16-byte aligned");
-    const int64_t rows = (n + kDequantRows - 1) / kDequantRows, groups = (blocks + kDequantBlocks - 1) / kDequantBlocks;
-    MAMBO_REQUIRE(rows <= 0x7FFFFFFF / groups, MAMBO_ERR_VALUE, "weight too large");
-    MAMBO_LAUNCH(dequant_kernel, dim3((unsigned)(rows * groups)), dim3(256), 0, (hipStream_t)stream, d, qs, qh, signs,
-                 scales, n, blocks, (uint32_t)groups, values, out_scales);
-    return mambo_check_launch("iq3s_dequant");
+    // 32 x 4 from 8 M weights; below, its few workgroups of long threads take longer than those of one
+    // store each (us, 16 x 1 and 32 x 4, a thread per group before: 512 x 2048 2.6, 3.7 and 2.8, 1024 x
+    // 4096 3.5, 4.1 and 4.1, 2048 x 4096 4.6, 4.5 and 5.6, 4096 x 4096 6.7, 6.0 and 8.8)
+    const auto launch = n <= 32767 / blocks ? launch_dequant<16, 1> : launch_dequant<32, 4>;
+    return launch(d, qs, qh, signs, scales, n, blocks, values, out_scales, (hipStream_t)stream);
 }

@@ -1,5 +1,5 @@
 """Weight preparation and decoding at the edges of their workgroups (64 rows x 4 blocks or a tile;
-32 rows x 4 blocks), from every form of source: whole fields against numpy, bit for bit,
+32 rows x 4 blocks or 16 x 1), from every form of source: whole fields against numpy, bit for bit,
 and the tile layout against the one that the byte path builds."""
 
 from __future__ import annotations
@@ -88,9 +88,11 @@ def test_prepare_of_repeated_rows(gpu):
     assert torch.equal(a.packed, b.packed) and torch.equal(a.signs, b.signs) and torch.equal(a.d, b.d)
 
 
-@pytest.mark.parametrize("n,blocks", [(1, 1), (31, 3), (33, 4), (64, 5), (100, 9)])
+# (16 rows x 1 block up to 32767 blocks, 32 x 4 from there)
+@pytest.mark.parametrize("n,blocks", [(1, 1), (31, 3), (33, 4), (64, 5), (100, 9), (32767, 1), (16384, 2), (33, 993),
+                                      (8193, 5), (31, 1059)])
 def test_dequant_into_scales_of_any_float_alignment(gpu, n, blocks):
-    """Edges of the decoder's 32 rows x 4 blocks, the scales four bytes off a 16-byte boundary, and
+    """Edges of the decoder's workgroups, the scales four bytes off a 16-byte boundary, and
     nothing written outside either output."""
     from mambo_amd import _native
     from mambo_amd.utils.iq3_s_weight import prepare_iq3_s_fields

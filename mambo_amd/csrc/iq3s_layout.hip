@@ -390,10 +390,12 @@ extern "C" int mambo_iq3s_prepare(const uint8_t *raw, int64_t n, int64_t blocks,
     MAMBO_REQUIRE(tiles <= 0x7FFFFFFF, MAMBO_ERR_VALUE, "N too large");
     // Contiguous blocks, fields that take the vector stores, and work for three quarters of the
     // 256 CUs: fields and tiles of 4096 x 4096 (256 workgroups) take 11.5 us here and 13.4 us a
-    // tile per workgroup, those of 1024 x 8192 or 2048 x 4096 (128) 8.1 and 7.5.
+    // tile per workgroup, those of 1024 x 8192 or 2048 x 4096 (128) 8.1 and 7.5. With one to three
+    // blocks a row a workgroup has that share of its work: 19473 x 256 (305) 9.1 and 7.3, 12288 x
+    // 512 (192) 8.9 and 7.6, 19473 x 512 (305) 10.3 and 11.0, 57344 x 256 (896) 10.6 and 13.1.
     const int64_t row_groups = (n + kPrepRows - 1) / kPrepRows, groups = (blocks + kPrepBlocks - 1) / kPrepBlocks;
-    if (stride_byte == 1 && stride_b == kIq3sBlockBytes && row_groups * groups >= 192 && (uintptr_t)qs % 16 == 0 &&
-        (uintptr_t)signs % 16 == 0 && (uintptr_t)qh % 8 == 0) {
+    if (stride_byte == 1 && stride_b == kIq3sBlockBytes && row_groups * groups >= 192 && row_groups * blocks >= 600 &&
+        (uintptr_t)qs % 16 == 0 && (uintptr_t)signs % 16 == 0 && (uintptr_t)qh % 8 == 0) {
         const dim3 grid((unsigned)row_groups, (unsigned)(groups < 65535 ? groups : 65535));
         MAMBO_LAUNCH(prepare_rows_kernel, grid, dim3(256), 0, (hipStream_t)stream, raw, stride_n, n, blocks, out);
     } else {

@@ -51,7 +51,8 @@ def sources(raw, gpu):
 
 @pytest.mark.parametrize("n,blocks", [
     (1, 1), (16, 2), (45, 5),  # a tile per workgroup
-    (1, 768), (65, 383), (192, 254), (12225, 1), (1100, 61)])  # 64 rows x 4 blocks: from 192 workgroups on
+    # 64 rows x 4 blocks: from 192 workgroups on whose rows hold 600 blocks together
+    (1, 768), (65, 383), (192, 254), (12225, 1), (1100, 61), (38337, 1), (13000, 3)])
 def test_prepare_forms_agree(gpu, n, blocks):
     from mambo_amd.kernels.iq3_s_fp8 import launch_dequant_iq3_s
     from mambo_amd.utils.iq3_s_weight import IQ3SFields, ensure_packed, prepare_iq3_s_fields

@@ -400,7 +400,7 @@ def test_tiled_kernel_every_tile_shape(gpu, m):
 
 @pytest.mark.parametrize("n,k", [(4096, 4096), (4096, 14336)])
 def test_prefill_shape_sampled(gpu, n, k):
-    """M=2048 prefill on 8B shapes (default config: the tiled kernel), sampled output
+    """M=2048 prefill on 8B shapes (default config: the 32 x 32 MFMA kernel), sampled output
     columns against the oracle."""
     from mambo_amd.kernels.iq3_s_fp8 import launch_iq3_s_fp8_matmul
     from mambo_amd.kernels.quantize_fp8 import launch_quantize_fp8

@@ -347,7 +347,7 @@ def points_report(args) -> None:
         lines += ["", "## MFMA counters (one eager step of each MFMA-bound point)", "", "Command:", "", "```",
                   args.mfma_command, "```", "",
                   f"MFMA busy = SQ_VALU_MFMA_BUSY_CYCLES / (GRBM_GUI_ACTIVE / {args.xcds} XCDs x "
-                  f"{args.cus * SIMD_PER_CU} SIMDs), over the step's tiled-kernel dispatches weighted by their "
+                  f"{args.cus * SIMD_PER_CU} SIMDs), over the step's dispatches weighted by their "
                   "active cycles; executed F8 flops = SQ_INSTS_VALU_MFMA_MOPS_F8 x 512.", "",
                   "| point | MFMA busy | executed / algorithmic F8 flops |", "|---|---|---|"]
         simds = args.cus * SIMD_PER_CU

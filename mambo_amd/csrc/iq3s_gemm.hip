@@ -1956,10 +1956,11 @@ int zero_outputs(const GroupArgs &ga, int64_t m, hipStream_t s)
     return mambo_check_launch("zero_rows");
 }
 
-// At least what a dense or unsplit tiled configuration takes (us; measured on the shapes of small_tiles):
+// About what a dense or unsplit tiled configuration takes (us; measured on the shapes of small_tiles):
 // a dense kernel that splits K 7 us with its zero fill and 1.5 us per 100 M multiply-adds; else the
 // chain of a wave's blocks (0.44 us each up to 16 tokens, 0.8 with 32 per workgroup, 1.25 in the tiled kernel's
-// 64 x 128 tiles) or the decodes of the dense kernel's 16 rows x 32 tokens (0.8 to 1.4 ns each).
+// 64 x 128 tiles) or the decodes of the dense kernel's 16 rows x 32 tokens (0.8 to 1.4 ns each; four waves
+// on large weights take 0.45 to 0.6 up to 16 tokens, which small_tiles allows for at its end).
 double config_time(const mambo_gemm_config &c, int64_t m, int64_t n, int64_t blocks)
 {
     if (c.kernel == MAMBO_GEMM_TILED)
@@ -1978,9 +1979,12 @@ double config_time(const mambo_gemm_config &c, int64_t m, int64_t n, int64_t blo
 //
 // True and the configuration where that is faster than what else takes the call, in other_us
 // microseconds (0: not known). Between 17 and 32 tokens the 32 x 64 tiles of that range stay. us
-// before and after: 4096 x 4096 at 48 / 128 tokens 11.6 -> 8.9, 17.4 -> 12.4; 1024 x 4096 10.5 -> 6.9 at
-// both; 2048 x 2816 at 128 16.8 -> 7.6; 4096 x 14336 at 48 27 -> 21; 8192 x 28672 at 48 73 -> 60; 640 x 3328
-// at 10 10.0 -> 5.5; 1314 x 18688 at 18 36 -> 15; geometric mean of 290 random shapes at 33 to 400 tokens 0.74.
+// before and after: 4096 x 4096 at 48 / 128 tokens 11.7 -> 9.2, 17.0 -> 12.6; 1024 x 4096 10.3 -> 6.0,
+// 10.5 -> 7.6; 2048 x 2816 at 128 22.7 -> 8.0; 4096 x 14336 at 48 27.5 -> 22.0; 8192 x 28672 at 48 78 ->
+// 73; 640 x 3328 at 10 9.7 -> 5.3; 1314 x 18688 at 18 36 -> 15. Both rules together, 480 random shapes:
+// geometric mean 0.74 at 5 to 10 tokens, 0.79 to 32, 0.73 at 33 to 400; the slowest ones against before:
+// 43453 x 512 at 47 13.1 -> 13.9, at 5 and 6 tokens 32-row tiles on 32 blocks and more (9914 x 16384
+// 26.7 -> 28.3, 8192 x 8192 10.9 -> 11.5).
 bool small_tiles(int64_t m, const mambo_projection *proj, int count, int64_t blocks, const uint8_t *xs, int64_t ldxs,
                  const mambo_gemm_config &other, double other_us, mambo_gemm_config *out)
 {

@@ -22,26 +22,29 @@
 // block's 16*MT f32 scalings are spread over the last and the next block's first step. The
 // packed words of the next block are requested as soon as their registers' last code is
 // decoded (a second block in flight measured no faster). 233 to 244 VGPRs at MT = 4, so two waves
-// per SIMD; what bounds it there is the power limit (1.7 GHz at 55% MFMA busy at 8192 tokens)
-// and, up to a few hundred tokens, the latency of a step's dependent chain.
+// per SIMD. What bounds it there is both the clock, which falls to 1.9 of 2.4 GHz under these MFMAs
+// (1.83 to 1.94 by GRBM_GUI_ACTIVE over launches of 0.3 ms and more), and the third of the MFMA cycles
+// that stay idle (60-69% busy at 8192 tokens, 67% on the 70B gate/up at 512; the waves wait for LDS,
+// memory or the barrier for 19-30% of their cycles and to issue for 32-38%): 2.45 to 2.67 PFLOP/s
+// executed, half of it useful. Up to a few hundred tokens it is the latency of a step's dependent chain.
 //
 // Two K groups (their sums meet in LDS at the end) put two waves on each SIMD where a launch
 // has a workgroup per CU or less: one wave leaves its SIMD idle while a step's chain of LDS
 // reads, decode and MFMAs completes (1.26 us a block of 64 tokens against 1.82 for two waves'),
 // and a K split over half as many workgroups costs half the atomics. One group against two,
-// each at its fastest split (us): 28672 x 4096 at 48 tokens 29 -> 25.6, 10240 x 8192 at 256
-// 59 -> 51, 6144 x 4096 at 256 25 -> 22, 8192 x 28672 at 128 80 -> 72, 4096 x 14336 at 256
-// 54 -> 43. Launches that fill the chip gain nothing from it (57344 x 8192 at 48: 82 and 85).
+// each at its fastest split (us): 28672 x 4096 at 48 tokens 29.3 -> 26.2, 10240 x 8192 at 256
+// 59 -> 57, 6144 x 4096 at 256 25.9 -> 22.7, 8192 x 28672 at 128 75 -> 72, 4096 x 14336 at 256
+// 45.4 -> 44.7. Launches that fill the chip gain nothing from it (57344 x 8192 at 48: 82 and 85).
 // Four groups of two waves (64 x 64 tiles) where even that leaves CUs without a workgroup: 8192 x
-// 8192 at 96 and 128 tokens 29 -> 26 and 31 -> 27, 6144 x 4096 18 -> 15.5 and 19 -> 16.
+// 8192 at 96 and 128 tokens 30.4 -> 27.6 and 32.8 -> 28.2, 6144 x 4096 18.3 -> 16.0 and 19.7 -> 16.2.
 // One 32-token sub-tile (MT = 1, reads a K step ahead) was built too and is level with the tiled
 // and dense kernels at 8 to 32 tokens (57344 x 8192 at 16 / 32 63 and 70 us against 54 and 70, 28672
 // x 4096 18 and 20 against 17 and 20): left out.
 //
 // Measured against the kernels it takes over from, same box, one launch in a replayed graph
-// over rotated weights (us): 57344 x 8192 at 40 / 128 / 512 tokens 133 -> 77, 133 -> 109, 456 ->
-// 398; 10240 x 8192 at 512 112 -> 90; 8192 x 28672 at 40 / 192 / 512 77 -> 43, 140 -> 102, 230 ->
-// 201; 28672 x 4096 at 2048 441 -> 401; 6204 x 2816 at 128 26 -> 18; 1280 x 8192 at 64 16 -> 12.
+// over rotated weights (us): 57344 x 8192 at 40 / 128 / 512 tokens 140 -> 87, 144 -> 122, 504 ->
+// 420; 10240 x 8192 at 256 / 512 65 -> 56, 113 -> 87; 8192 x 28672 at 128 / 192 / 512 86 -> 73, 149 ->
+// 114, 247 -> 210; 28672 x 4096 at 40 / 2048 29.5 -> 25.4, 476 -> 414; 6204 x 2816 at 128 27 -> 14.
 #include "iq3s_wide.h"
 #include "iq3s_wide_copies.h"
 
@@ -449,8 +452,10 @@ constexpr int64_t kCUs = 256;
 // K in `splits` slices: the busiest CU's rounds, the output stores, and with several slices
 // the zero fill and the f32 atomics (~1.5 TB/s alone). One K group fitted to 12000 launches (42
 // shapes of 128 to 57344 rows, K 512 to 28672, 33 to 4096 tokens, each at every shape and split;
-// rms error 6%), two to 250; the plan it picks is 1% behind the fastest measured one on average
-// over 66 shapes and token counts (most: 8%, 8192 x 4096 at 64 tokens).
+// rms error 6%), two to 250, four to the launches named above only; the plan it picks is 1% behind the
+// fastest measured one on average over 66 shapes and token counts (most: 8%, 8192 x 4096 at 64 tokens).
+// Large launches at 128 tokens lie outside that error: 57344 x 8192 takes 102 to 122 us where it says
+// 91, 8192 x 28672 62 to 73 where it says 56.
 double wide_time(const WideShape &w, int64_t wgs, int64_t b, int splits, double mb)
 {
     b = cdiv(b, w.kg);
@@ -503,9 +508,10 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
     // where 128 x 128 tiles give every CU one, but on 4 blocks not where the other's 64 x 128 tiles are
     // a single round of two per CU (8192 x 1024 at 400 tokens 13.1 and 14.7); against the dense kernel (which decodes a weight
     // once per 32 tokens) where 64 x 128 tiles take 80 CUs (us at 40 tokens: 28672
-    // x 4096 46 against 25, 14336 x 8192 43 and 36, 10240 x 4096 21.3 and 20.1; 8192 x 4096,
+    // x 4096 46 against 25, 14336 x 8192 42 and 29, 10240 x 4096 22 and 16; 8192 x 4096,
     // 64 workgroups, 16.3 and 19.9), or where its waves do not divide few K blocks and it takes 64
-    // rows a workgroup (6144 x 2816 23 against 16; with 32 rows, 4096 x 2816, 13.4 and 16.2).
+    // rows a workgroup (measured at 11 blocks, K = 2816, alone: 6144 rows 23 against 16; with 32 rows,
+    // 4096, 13.4 and 16.2; the small tiles take most of these launches from either).
     const bool split = blocks > cdiv(blocks, other.split_k);
     const int64_t row_wgs = wide_workgroups(proj, count, 4);
     const bool fills = row_wgs * cdiv(m, 128) >= kCUs;

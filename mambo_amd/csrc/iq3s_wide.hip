@@ -525,15 +525,17 @@ bool mambo_wide_plan(int64_t m, const mambo_projection *proj, int count, int64_t
     const double mb = 4e-6 * (double)m * (double)n;
     double best = 0.0;
     for (const WideShape &w : kWideShapes) {
-        // eight waves from 9 blocks on: four of them on 128 x 128 tiles are 4-17% faster before
-        // (7383 x 1280 at 959 tokens 30.6 and 25.6, 22818 x 2048 at 921 112 and 102)
-        if (w.waves == 8 && blocks < 9)
-            continue;
         // 64-token tiles decode each weight twice as often: only while 128-token ones leave CUs
         // idle, or where they pad away most of the last tile
         if (w.mt == 2 && fills && (m % 128 == 0 || m % 128 > 64))
             continue;
         const int64_t wgs = wide_workgroups(proj, count, w.waves) * cdiv(m, 32 * w.mt);
+        // on fewer than 9 blocks eight waves only where four would just pass one workgroup per CU (13208 x
+        // 1536 at 384 tokens, 156 workgroups, 24.8 us and 25.9 with four); else four of them on 128 x 128
+        // tiles are 4-17% faster (7383 x 1280 at 959, 232, 30.6 and 25.6; 22818 x 2048 at 921, 720,
+        // 112 and 102)
+        if (w.waves == 8 && blocks < 9 && wgs > kCUs * 11 / 16)
+            continue;
         if (wgs > 0x7FFFFFFF)
             return false;
         for (const int s : kWideSplits) {

@@ -46,7 +46,7 @@ def project(gpu, xv, xs, raws, config=None, pad=0):
 # slices of one and of several blocks with a short last one, last 16-row tile alone in its pair, tokens
 # one past and one short of a tile, one to all of a tile's rows padded
 SHAPES = [(1000, [4090], 4, (4, 4, 2, 1)), (1025, [3000, 1100], 5, (2, 4, 1, 1)), (961, [8190], 5, (4, 4, 1, 1)),
-          (1024, [8000, 190], 4, (4, 4, 1, 1)), (450, [8208], 4, (4, 4, 1, 1)), (2048, [16000], 4, (4, 4, 1, 1)),
+          (1024, [8000, 190], 4, (4, 4, 1, 1)), (450, [8208], 4, (4, 8, 1, 1)), (2048, [16000], 4, (4, 4, 1, 1)),
           (48, [57344], 4, (2, 4, 1, 1)), (338, [11079], 9, (4, 8, 1, 1)), (1000, [8190], 10, (4, 8, 1, 1)),
           (129, [8192], 13, (2, 4, 2, 1)), (76, [10895, 18], 9, (2, 4, 2, 1)), (146, [11106], 9, (4, 4, 2, 1)),
           (35, [8882], 7, (2, 2, 4, 1)), (718, [2], 10, (2, 2, 4, 1)), (128, [4100, 4000], 23, (2, 2, 4, 1)),

@@ -81,5 +81,6 @@ def test_plan_where_the_named_default_is_the_faster():
     # four K blocks where 64-token tiles are one round of two workgroups per CU
     assert plan(400, [8192], 4) == {"kernel": tiled, "waves": 8, "split_k": 1, "tile_m": 64, "tile_n": 128}
     assert plan(400, [10240], 4)["kernel"] == wide and plan(400, [8192], 5)["kernel"] == wide
-    # eight waves of 32 rows from nine K blocks
-    assert plan(960, [7383], 8)["tile_n"] == 128 and plan(960, [28672], 9)["tile_n"] == 256
+    # eight waves of 32 rows from nine K blocks, and on fewer where four would just pass a workgroup per CU
+    assert plan(959, [7383], 5)["tile_n"] == 128 and plan(960, [28672], 9)["tile_n"] == 256
+    assert plan(384, [13208], 6)["tile_n"] == 256

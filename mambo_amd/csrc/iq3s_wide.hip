@@ -176,8 +176,16 @@ __global__ __launch_bounds__(W * KG * 64) __attribute__((amdgpu_waves_per_eu(2))
                    od = second + 2u * col;
 
     // Rows past M read row M-1 (their outputs are never stored), by offsets made once
-    // (iq3s_wide_copies.h).
-    const __amdgpu_buffer_rsrc_t xrows = byte_rsrc(xv + m0 * ldxv), srows = byte_rsrc(xs + m0 * ldxs);
+    // (iq3s_wide_copies.h). The resources end with that row too; nothing depends on it, but with open ones the
+    // compiler's code around the stores is slower where N is no multiple of 16 (2286 x 2048 at 1920 tokens
+    // 28.0 us and 27.4, 2897 x 1024 at 1536 18.5 and 17.9).
+    const auto rows_rsrc = [&](const uint8_t *base, int64_t ld, int row_bytes) {
+        const uint64_t bytes = (uint64_t)(M - 1 - m0) * (uint64_t)ld + (uint64_t)row_bytes;
+        const uint32_t n = (bytes >> 32) ? 0xFFFFFFFFu : (uint32_t)bytes;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base + m0 * ld), 0,
+                                                 __builtin_amdgcn_readfirstlane((int)n), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t xrows = rows_rsrc(xv, ldxv, B * 256), srows = rows_rsrc(xs, ldxs, B * 8);
     const int last_row = (int)min<int64_t>(M - 1 - m0, kRows - 1);
     const int srow = wave & (MT - 1); // waves past MT repeat a scale copy (the same bytes): no branch
     uint32_t voff[kVCopies];
